@@ -22,10 +22,19 @@ struct MmArgs {
     int64_t w_nb1, x_nb1, d_nb1;
     int32_t M, N, K;
     int32_t tiles_m, tiles_n, n_blocks;
+    int32_t cols;        // mm_ksplit: output tiles per column of the tile order
 };
 
 // Enqueue the product (x F32 when x_f32, else BF16).
 hipError_t launch_mm(const MmArgs &a, bool x_f32, hipStream_t stream);
+
+// Enqueue the few-token kernels (kd_mm_ksplit.hip): mm_skinny (M <= 16), and
+// mm_ksplit with tiles of 32 * (tile / 10) outputs x 32 * (tile % 10) tokens
+// (tile 11, 21, 22, 23, 42, 43 or 44); they count their own tiles.
+constexpr int kMmSkinnyRows = 16;
+constexpr int64_t kMmMaxBlocks = 1 << 23;   // workgroups of 256 threads in one launch, with room to spare
+hipError_t launch_mm_skinny(const MmArgs &a, bool x_f32, hipStream_t stream);
+hipError_t launch_mm_ksplit(const MmArgs &a, int tile, bool x_f32, hipStream_t stream);
 
 struct DqArgs {
     const char *w;       // weight rows [N], row stride w_nb1 bytes

@@ -1,0 +1,58 @@
+"""The few-token kernels of the linear-layer product (kd_mm_ksplit.hip)
+against the float64 product of the same BF16-rounded operands: tokens at and
+past every boundary of the kernel choice and of the tiles, outputs that end
+inside a tile, k of one half stage, whole stages, a half last one and more
+stages than the LDS rings hold, rows with padding behind them."""
+import numpy as np
+import pytest
+import torch
+
+import kd_mm
+import kd_oracle_quant as oq
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+# M, N, K; the tile the choice takes stands beside the larger ones
+CASES = [(1, 4, 32), (8, 36, 96), (9, 100, 416), (16, 260, 1184), (3, 16388, 288), (12, 16384, 64),
+         (17, 32, 64), (33, 100, 544),
+         (31, 8200, 160),     # 64 x 32
+         (130, 4100, 96),     # 64 x 64
+         (300, 4096, 416),    # 64 x 96
+         (850, 2100, 672),    # 128 x 64
+         (700, 4100, 352),    # 128 x 96
+         (1030, 8000, 736),   # 128 x 128
+         (2049, 4064, 352)]
+
+
+@pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
+def test_few_tokens(case, xdt):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    M, N, K = case
+    print(f"[case] mm {case} {xdt}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    # rows of a wider matrix: what lies behind a row is never part of it
+    w = torch.full((N, K + 8), float("nan"), dtype=torch.bfloat16)
+    w[:, :K] = torch.randn((N, K), generator=g) * 0.05
+    x = torch.full((M, K + 8), float("nan"), dtype=xdt)
+    x[:, :K] = torch.randn((M, K), generator=g)
+    bias = torch.randn(N, generator=g) * 0.1 if N % 8 else None
+    out = torch.full((M + 1, N + 4), 7.0, device=DEV)
+    d = kd_mm.make_desc(w.to(DEV)[:, :K], x.to(DEV)[:, :K], None if bias is None else bias.to(DEV), out[:M, :N])
+    assert kd_mm.run_desc(d) == 0
+    torch.cuda.synchronize()
+    wr = w[:, :K].double()
+    xr = torch.from_numpy(oq.round_bf16(x[:, :K].float().numpy())).double()
+    ref = xr @ wr.T + (0.0 if bias is None else bias.double())
+    # F32 accumulation of K products in any order: K rounding errors of 2^-24 of the sum of magnitudes at most
+    limit = (xr.abs() @ wr.abs().T + (0.0 if bias is None else bias.double().abs())) * (K + 8) * 2.0 ** -24 + 1e-30
+    got = out.cpu()
+    err = (got[:M, :N].double() - ref).abs()
+    assert bool((err <= limit).all()), float((err / limit).max())
+    assert bool((got[M:] == 7.0).all()) and bool((got[:, N:] == 7.0).all())
+    assert kd_mm.run_desc(d) == 0
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy(), got.numpy())
