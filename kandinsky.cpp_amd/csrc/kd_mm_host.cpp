@@ -100,21 +100,22 @@ size_t ws_bytes(const kd_mm_desc *d) {
     return w_direct(d->w) ? 0 : (size_t)d->w.ne[0] * (size_t)d->w.ne[1] * 2;
 }
 
-// The kernel of a call: mm_skinny up to 16 tokens; else the tile whose rounds
-// of workgroups (256 at once, one per CU) take least time: 0 for mm_bf16's
-// 256 x 256, else mm_ksplit's.  `us` is a tile's time per round with every CU
-// at it, K = 4096 and F32 x (all scale with K, and by 0.7-0.84 with BF16 x,
-// so their order holds): small tiles move more bytes per product, large ones
+// The tile of a call (32 * (tile / 10) outputs x 32 * (tile % 10) tokens) of
+// more than kMmSkinnyRows tokens: the one whose rounds of workgroups (256 at
+// once, one per CU) take least time.  `us` is a round's time with every CU at
+// it, K = 4096 and F32 x (all scale with K, and by 0.7-0.9 with BF16 x, so
+// their order holds): small tiles move more bytes per product, large ones
 // leave CUs idle.
 int choose_tile(int64_t M, int64_t N) {
     constexpr struct { int tile, n, m; double us; } kTiles[] = {
-        {0, 256, 256, 140.0}, {44, 128, 128, 43.0}, {43, 128, 96, 36.0}, {42, 128, 64, 27.5},
-        {23, 64, 96, 27.0},   {22, 64, 64, 19.0},   {21, 64, 32, 12.5},  {11, 32, 32, 9.0}};
-    int best = 0;
+        {88, 256, 256, 122.0}, {84, 256, 128, 76.0}, {44, 128, 128, 43.0}, {43, 128, 96, 36.0},
+        {42, 128, 64, 27.5},   {23, 64, 96, 27.0},   {22, 64, 64, 19.0},   {21, 64, 32, 12.5},
+        {11, 32, 32, 9.0}};
+    int best = 88;
     double least = 1e300;
     for (const auto &t : kTiles) {
         const int64_t tiles = ((N + t.n - 1) / t.n) * ((M + t.m - 1) / t.m);
-        if (t.tile && tiles > kdfa::kMmMaxBlocks) continue;
+        if (t.tile != 88 && tiles > kdfa::kMmMaxBlocks) continue;
         const double cost = (double)((tiles + 255) / 256) * t.us;
         if (cost < least) { least = cost; best = t.tile; }
     }
@@ -190,15 +191,16 @@ int kd_mm_run(const kd_mm_desc *desc, void *workspace, size_t workspace_bytes, v
     a.M = (int32_t)M;
     a.N = (int32_t)N;
     a.K = (int32_t)K;
-    a.tiles_m = (int32_t)((M + kdfa::kMmBM - 1) / kdfa::kMmBM);
-    a.tiles_n = (int32_t)((N + kdfa::kMmBN - 1) / kdfa::kMmBN);
-    if ((int64_t)a.tiles_m * a.tiles_n > kI32Max) return KD_FA_ERR_SHAPE;
-    a.n_blocks = a.tiles_m * a.tiles_n;
+    if (((M + kdfa::kMmBM - 1) / kdfa::kMmBM) * ((N + kdfa::kMmBN - 1) / kdfa::kMmBN) > kI32Max) return KD_FA_ERR_SHAPE;
+    a.tiles_m = a.tiles_n = a.n_blocks = a.cols = 0;
     const bool x_f32 = desc->x.type == KD_MM_TYPE_F32;
-    const int tile = M <= kdfa::kMmSkinnyRows && N <= 32 * kdfa::kMmMaxBlocks ? -1 : choose_tile(M, N);
-    const hipError_t e = tile < 0    ? kdfa::launch_mm_skinny(a, x_f32, hs)
-                         : tile == 0 ? kdfa::launch_mm(a, x_f32, hs)
-                                     : kdfa::launch_mm_ksplit(a, tile, x_f32, hs);
+    hipError_t e;
+    if (M <= kdfa::kMmSkinnyRows && N <= 32 * kdfa::kMmMaxBlocks) {
+        e = kdfa::launch_mm_skinny(a, x_f32, hs);
+    } else {
+        const int tile = choose_tile(M, N);
+        e = tile == 88 || tile == 84 ? kdfa::launch_mm(a, tile, x_f32, hs) : kdfa::launch_mm_ksplit(a, tile, x_f32, hs);
+    }
     return e == hipSuccess ? KD_FA_OK : KD_FA_ERR_LAUNCH;
 }
 

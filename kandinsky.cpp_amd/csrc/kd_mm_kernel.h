@@ -8,8 +8,8 @@
 
 namespace kdfa {
 
-// Workgroup tile of the product: 256 rows of x (tokens) by 256 rows of w
-// (outputs), 32 k per stage.
+// Largest workgroup tile of the product: 256 rows of x (tokens) by 256 rows
+// of w (outputs), 32 k per stage.
 constexpr int kMmBM = 256;
 constexpr int kMmBN = 256;
 constexpr int kMmBK = 32;
@@ -21,16 +21,18 @@ struct MmArgs {
     char *dst;           // F32 rows [M][N], row stride d_nb1 bytes
     int64_t w_nb1, x_nb1, d_nb1;
     int32_t M, N, K;
-    int32_t tiles_m, tiles_n, n_blocks;
-    int32_t cols;        // mm_ksplit: output tiles per column of the tile order
+    // set by the launchers: the tiles, and the output tiles per column of
+    // their order
+    int32_t tiles_m, tiles_n, n_blocks, cols;
 };
 
-// Enqueue the product (x F32 when x_f32, else BF16).
-hipError_t launch_mm(const MmArgs &a, bool x_f32, hipStream_t stream);
+// Enqueue the product (x F32 when x_f32, else BF16) with tiles of 256 outputs
+// x 256 (tile 88) or 128 tokens (84).
+hipError_t launch_mm(const MmArgs &a, int tile, bool x_f32, hipStream_t stream);
 
 // Enqueue the few-token kernels (kd_mm_ksplit.hip): mm_skinny (M <= 16), and
 // mm_ksplit with tiles of 32 * (tile / 10) outputs x 32 * (tile % 10) tokens
-// (tile 11, 21, 22, 23, 42, 43 or 44); they count their own tiles.
+// (tile 11, 21, 22, 23, 42, 43 or 44).
 constexpr int kMmSkinnyRows = 16;
 constexpr int64_t kMmMaxBlocks = 1 << 23;   // workgroups of 256 threads in one launch, with room to spare
 hipError_t launch_mm_skinny(const MmArgs &a, bool x_f32, hipStream_t stream);

@@ -5,17 +5,15 @@
 //                   one 32-element block per thread, in the F32 arithmetic
 //                   of ggml's dequantize_row_q4_0 / _q8_0
 //   mm_bf16         dst[m][n] = sum_k w[n][k] x[m][k] (+ bias[n]) on
-//                   v_mfma_f32_32x32x16_bf16, F32 accumulation
+//                   v_mfma_f32_16x16x32_bf16, F32 accumulation
 //
 // The product computes D^T = W X^T: A = W (outputs on M), B = X^T (tokens
 // on N), so that each lane ends with 4 consecutive outputs of one token --
 // 16-byte pieces of a dst row.  Both operands are k-contiguous rows, which
-// is exactly the MFMA operand form (A: lane l holds row l%32, k 8*(l/32)..
-// +7; B: column l%32, the same k) -- no transposes anywhere.
+// is exactly the MFMA operand form (A: lane l holds row l%16, k 8*(l/16)..
+// +7; B: column l%16, the same k) -- no transposes anywhere.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-
-#include <type_traits>
 
 #include "../../include/kd_mm.h"
 #include "kd_fa_device.h"
@@ -110,270 +108,270 @@ hipError_t launch_dequant(const DqArgs &a, hipStream_t s) {
 
 // ---------------------------------------------------------------------------
 // mm_bf16: one workgroup = 4 waves (one per SIMD, 512 registers each) = a
-// 256 (outputs) x 256 (tokens) tile of dst; wave w holds the 128 x 128
-// quarter (w & 1, w >> 1) as 4 x 4 MFMA accumulator blocks (256 AGPRs).
+// 256 (outputs) x 64 MB (tokens) tile of dst; wave w holds the 128 x 32 MB
+// quarter (w & 1, w >> 1) as 8 x 2 MB accumulator blocks of 16 x 16 (256
+// AGPRs at MB = 4).
 //
-// K advances 32 per stage through S LDS stages (4 with BF16 X, 3 with F32
-// X: 128 / 144 KiB), each filled by DMA (global_load_lds_dwordx4) S - 1
-// stages ahead of its use:
-//   W stage: 256 rows x 64 bytes (BF16); 16-byte chunk c of row r at
-//            c ^ ((r >> 2) & 3)
-//   X stage: 256 rows x 128 bytes (F32) or 64 bytes (BF16); chunk c of row
-//            r at c ^ ((r >> 1) & 7) (F32) or c ^ ((r >> 2) & 3) (BF16)
-// -- so that the 16 rows one 16-lane group of an operand read touches fill
-// the 256 bytes of the 64 banks exactly once.  F32 X is rounded to BF16
-// next to the MFMAs that use its fragments.  Per stage a wave reads 8 W and
-// 8 X fragments and issues 32 MFMAs, with the DMAs of a later stage spread
-// over the first 16; the only barrier is the one that publishes a stage.
-// Rows past M or N read clamped (repeated) rows and are not stored; the
-// workgroups an XCD runs at once cover 8 token tiles x 4 output tiles, so
-// its L2 serves their shared W and X stages.  The output goes through LDS so
-// that its stores are whole 128-byte lines.
+// The products are v_mfma_f32_16x16x32_bf16: at full chip the power limit
+// sets the rate, and on random operands 16 x 16 x 32 sustains 1,995 TFLOP/s
+// against 1,700 for 32 x 32 x 16 (register operands only; on zeros 2,440 and
+// 2,480).
+//
+// K advances 32 per stage.  W (256 rows x 64 bytes) comes by DMA
+// (global_load_lds_dwordx4), kS - 1 stages ahead; BF16 X the same way, with
+// its stage.  F32 X is loaded into registers two stages ahead of its
+// rounding to BF16 and its way into one of two LDS buffers, so that it costs
+// the LDS the same as BF16 X: read from LDS as F32, X alone kept it busy for
+// 768 of a stage's 1,024 matrix cycles.  In LDS 16-byte chunk c of row r
+// lies at c ^ ((r >> 2) & 3): the 16 rows that 16 lanes of an operand read
+// touch fill the 64 banks once.  Per stage a wave reads 8 W and 2 MB X
+// fragments and issues 16 MB MFMAs in two halves (all W against half of X),
+// the DMAs of a later stage spread over the first, the loads, roundings and
+// LDS writes of X over the second; the one barrier, between them, publishes
+// the next stage.  The loop has no conditions: past the last stage the DMAs
+// and loads bring the last one again.
+// Rows past M or N read clamped (repeated) rows and are not stored.  The
+// output goes through LDS so that its stores are whole 128-byte lines.
 // ---------------------------------------------------------------------------
 constexpr int kMmWaves = 4;
 constexpr int kMmWTile = kMmBN * kMmBK * 2;   // 16 KiB
 
-template <bool XF32>
+template <bool XF32, int MB>
 __global__ __launch_bounds__(64 * kMmWaves) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void mm_bf16(MmArgs a) {
     typedef Elem<__bf16> E;
     typedef E::vec8 vec8;
-    constexpr int kXRow = XF32 ? 128 : 64;               // bytes of one X row per stage
-    constexpr int kXTile = kMmBM * kXRow;
-    constexpr int kStage = kMmWTile + kXTile;
-    constexpr int kThreads = 64 * kMmWaves;
-    constexpr int kWRounds = kMmWTile / (kThreads * 16);   // 4
-    constexpr int kXRounds = kXTile / (kThreads * 16);     // 8 (F32) or 4
-    constexpr int kWRowsPerRound = 1024 / 64;              // 16 rows per wave DMA
-    constexpr int kXRowsPerRound = 1024 / kXRow;           // 8 or 16
-    constexpr int kS = XF32 ? 3 : 4;                       // LDS stages
-    constexpr int kPer = kWRounds + kXRounds;              // DMAs per stage per wave
-    __shared__ __attribute__((aligned(1024))) char lds[kS * kStage];
+    constexpr int BM = 64 * MB;
+    constexpr int kXTile = BM * 64;                        // BF16 X rows of a stage
+    constexpr int kS = XF32 ? 6 : MB == 4 ? 5 : 6;         // stages of W (and BF16 X) in LDS
+        constexpr int kXC = 2 * MB;                            // F32 X: 16-byte loads of a thread per stage
+    constexpr int kXD = XF32 ? 0 : MB;                     // BF16 X: DMAs of a wave per stage
+    constexpr int kVm = 4 + (XF32 ? kXC : kXD);            // vector memory operations of a wave per stage
+    constexpr int kX0 = kS * kMmWTile;                     // the X buffers behind W's
+    constexpr int kUse = kX0 + (XF32 ? 2 : kS) * kXTile;
+    constexpr int kEpi = kMmWaves * 8192 * MB;             // two blocks of 32 outputs per wave
+    __shared__ __attribute__((aligned(1024))) char lds[kUse > kEpi ? kUse : kEpi];
     lds_t *const sbase = LDS_PTR(char, lds);
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l32 = lane & 31;
-    const int hi = lane >> 5;
+    const int l16 = lane & 15;
+    const int q4 = lane >> 4;
 
-    // tile: XCD-contiguous runs of tiles, dealt in columns of 4 output tiles
-    // (m fastest within a column): the 32 workgroups an XCD runs at once
-    // then share 4 W tiles and 8 X tiles in its L2, where n-fastest order
-    // (16 W, 2 X) spread them over more (3-8% at the DiT's shapes)
+    // tile: XCD-contiguous runs of tiles, dealt in columns of `cols` output
+    // tiles (token tiles one after another within a column): the 32
+    // workgroups an XCD runs at once then share 4 W tiles and 8 X tiles in
+    // its L2
     const int pid = blockIdx.x;
     const int per = a.n_blocks >> 3;
     const int lid = pid < per * 8 ? (pid & 7) * per + (pid >> 3) : pid;
-    int nt, mt;
-    if (a.tiles_n % 4 == 0) {
-        const int col = lid / (a.tiles_m * 4), rem = lid % (a.tiles_m * 4);
-        mt = rem / 4;
-        nt = col * 4 + rem % 4;
-    } else {
-        nt = lid % a.tiles_n;
-        mt = lid / a.tiles_n;
-    }
-    const int n0 = nt * kMmBN;
-    const int m0 = mt * kMmBM;
+    const int col = lid / (a.tiles_m * a.cols), rem = lid - col * (a.tiles_m * a.cols);
+    const int width = min(a.cols, a.tiles_n - col * a.cols);
+    const int mt = rem / width;
+    const int n0 = (col * a.cols + rem - mt * width) * kMmBN;
+    const int m0 = mt * BM;
 
-    // DMA lane offsets, relative to the tile's first row (the stage base
-    // moves by 64 / kXRow bytes per stage)
-    uint32_t w_off[kWRounds], x_off[kXRounds];
+    // DMA lane offsets, relative to the tile's first row
+    uint32_t w_off[4], xd_off[XF32 ? 1 : MB], x_off[kXC];
+    const int dr = lane >> 2, dc = (lane & 3) ^ ((lane >> 4) & 3);   // chunk dc of row 16 i + dr
 #pragma unroll
-    for (int j = 0; j < kWRounds; ++j) {
-        const int r = kWRowsPerRound * (wave + kMmWaves * j) + (lane >> 2);
-        const int c = (lane & 3) ^ ((r >> 2) & 3);
-        const int rr = n0 + r < a.N ? r : a.N - 1 - n0;
-        w_off[j] = (uint32_t)rr * (uint32_t)a.w_nb1 + (uint32_t)(c << 4);
-    }
+    for (int j = 0; j < 4; ++j)
+        w_off[j] = (uint32_t)min(16 * (wave + kMmWaves * j) + dr, a.N - 1 - n0) * (uint32_t)a.w_nb1 + (uint32_t)(dc << 4);
+    if constexpr (XF32) {
+        // load j of a thread: 4 F32 of row 8 (wave + 4 j) + lane / 8, to
+        // x_wr + 2048 j of an X buffer
 #pragma unroll
-    for (int j = 0; j < kXRounds; ++j) {
-        const int r = kXRowsPerRound * (wave + kMmWaves * j) + (XF32 ? (lane >> 3) : (lane >> 2));
-        const int c = XF32 ? ((lane & 7) ^ ((r >> 1) & 7)) : ((lane & 3) ^ ((r >> 2) & 3));
-        const int rr = m0 + r < a.M ? r : a.M - 1 - m0;
-        x_off[j] = (uint32_t)rr * (uint32_t)a.x_nb1 + (uint32_t)(c << 4);
+        for (int j = 0; j < kXC; ++j) {
+            const int r = 8 * (wave + kMmWaves * j) + (lane >> 3);
+            x_off[j] = (uint32_t)min(r, a.M - 1 - m0) * (uint32_t)a.x_nb1 + (uint32_t)((lane & 7) << 4);
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < MB; ++j)
+            xd_off[j] = (uint32_t)min(16 * (wave + kMmWaves * j) + dr, a.M - 1 - m0) * (uint32_t)a.x_nb1 + (uint32_t)(dc << 4);
     }
+    const int xr = 8 * wave + (lane >> 3);
+    const uint32_t x_wr =
+        (uint32_t)(kX0 + xr * 64 + ((((lane & 7) >> 1) ^ ((xr >> 2) & 3)) << 4) + ((lane & 1) << 3));
     const char *const wtile = a.w + (int64_t)n0 * a.w_nb1;
     const char *const xtile = a.x + (int64_t)m0 * a.x_nb1;
-    // DMA j (of kPer) of stage kt into LDS stage buffer st: W rounds first
-    auto dma_j = [&](int kt, int st, int j) __attribute__((always_inline)) {
-        lds_t *sw = sbase + st * kStage;
-        if (j < kWRounds)
-            dma16(wtile + kt * 64, w_off[j], sw + (wave + kMmWaves * j) * 1024);
-        else
-            dma16(xtile + kt * kXRow, x_off[j - kWRounds], sw + kMmWTile + (wave + kMmWaves * (j - kWRounds)) * 1024);
+    const int nk = a.K / kMmBK;
+    // DMA j of stage kt (W's four, then BF16 X's) into buffer buf
+    auto dma_j = [&](int kt, int buf, int j) __attribute__((always_inline)) {
+        const int64_t k64 = (int64_t)min(kt, nk - 1) * 64;
+        if (j < 4)
+            dma16(wtile + k64, w_off[j], sbase + buf * kMmWTile + (wave + kMmWaves * j) * 1024);
+        else if constexpr (!XF32)
+            dma16(xtile + k64, xd_off[j - 4], sbase + kX0 + buf * kXTile + (wave + kMmWaves * (j - 4)) * 1024);
     };
-    auto issue = [&](int kt, int st) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < kPer; ++j) dma_j(kt, st, j);
+    f32x4 xs[2][kXC];
+    auto load_x = [&](int kt, int j, f32x4 &v) __attribute__((always_inline)) {
+        v = *reinterpret_cast<const f32x4 *>(xtile + (int64_t)min(kt, nk - 1) * 128 + x_off[j]);
+    };
+    auto write_x = [&](int buf, int j, const f32x4 &v) __attribute__((always_inline)) {
+        *reinterpret_cast<__attribute__((address_space(3))) u32x2 *>(sbase + x_wr + j * 2048 + buf * kXTile) =
+            (u32x2){E::pack2(v.x, v.y), E::pack2(v.z, v.w)};
     };
 
-    // fragment read offsets within a stage (the row part of the swizzle is
-    // l32's, since every block starts at a multiple of 32 rows)
+    // fragments: lane l holds row l % 16, k 8 * (l / 16) .. +7 of the stage
     const int wn = wave & 1;
     const int wm = wave >> 1;
-    uint32_t a_rd[2], b_rd[2][2];
+    const uint32_t f_rd = (uint32_t)(l16 * 64 + ((q4 ^ ((l16 >> 2) & 3)) << 4));
+    const uint32_t a_rd = f_rd + 128 * wn * 64;
+    const uint32_t b_rd = f_rd + kX0 + 32 * MB * wm * 64;
+    f32x4 acc[8][2 * MB];
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-        a_rd[ks] = (uint32_t)((128 * wn + l32) * 64 + (((2 * ks + hi) ^ ((l32 >> 2) & 3)) << 4));
-        if (XF32) {
-            b_rd[ks][0] = (uint32_t)(kMmWTile + (128 * wm + l32) * 128 + (((4 * ks + 2 * hi) ^ ((l32 >> 1) & 7)) << 4));
-            b_rd[ks][1] = (uint32_t)(kMmWTile + (128 * wm + l32) * 128 + (((4 * ks + 2 * hi + 1) ^ ((l32 >> 1) & 7)) << 4));
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 2 * MB; ++j) acc[i][j] = (f32x4){};
+    vec8 fa[2][8], fb[2][MB];
+    typedef const __attribute__((address_space(3))) vec8 lds_v8;
+    auto read_a = [&](int buf, auto p_c, int i) __attribute__((always_inline)) {
+        fa[decltype(p_c)::value][i] = *reinterpret_cast<lds_v8 *>(sbase + buf * kMmWTile + a_rd + i * 1024);
+    };
+    auto read_b = [&](int buf, auto h_c, int j) __attribute__((always_inline)) {
+        constexpr int h = decltype(h_c)::value;
+        fb[h][j] = *reinterpret_cast<lds_v8 *>(sbase + buf * kXTile + b_rd + (h * MB + j) * 1024);
+    };
+    // the products of W set p with half h of X; after product i, between(i)
+    auto products = [&](auto p_c, auto h_c, auto between) __attribute__((always_inline)) {
+        constexpr int p = decltype(p_c)::value, h = decltype(h_c)::value;
+#pragma unroll
+        for (int j = 0; j < MB; ++j)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][h * MB + j]) : "v"(fa[p][i]), "v"(fb[h][j]));
+                __builtin_amdgcn_sched_barrier(0);
+                between(8 * j + i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+    };
+
+    // The vector memory work of a stage interval (between two barriers), in
+    // two halves.  The first, while a step's second products run: stage dk's
+    // F32 X rounded from registers (set and buffer dk & 1 = xp) into LDS and
+    // the registers loaded for stage dk + 2, or the first DMAs of stage
+    // dk + kS - 2 into its buffer dbuf.  The second, while the next step's
+    // first products run: W's DMAs of stage dk + kS - 2, or the rest of them.
+    // (F32 x, 63,488 tokens: X and W mixed in both halves 2.20 ms against
+    // 2.06.)
+    constexpr int kWork0 = XF32 ? kXC : 2 + MB / 2, kWork1 = XF32 ? 4 : 2 + MB / 2;
+    auto work0 = [&](int slot, int dk, int dbuf, auto xp_c) __attribute__((always_inline)) {
+        constexpr int xp = decltype(xp_c)::value;
+        if constexpr (XF32) {
+            write_x(xp, slot, xs[xp][slot]);
+            load_x(dk + 2, slot, xs[xp][slot]);
         } else {
-            b_rd[ks][0] = (uint32_t)(kMmWTile + (128 * wm + l32) * 64 + (((2 * ks + hi) ^ ((l32 >> 2) & 3)) << 4));
-            b_rd[ks][1] = 0;
+            dma_j(dk + kS - 2, dbuf, slot);
+        }
+    };
+    auto work1 = [&](int slot, int dk, int dbuf) __attribute__((always_inline)) {
+        dma_j(dk + kS - 2, dbuf, XF32 ? slot : kWork0 + slot);
+    };
+#pragma unroll
+    for (int s = 0; s < kS - 1; ++s)
+#pragma unroll
+        for (int j = 0; j < 4 + kXD; ++j) dma_j(s, s, j);
+    if constexpr (XF32) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int j = 0; j < kXC; ++j) load_x(p, j, xs[p][j]);
+    }
+    // every stage issued so far has landed: the loop's first waits count on it
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (XF32) {
+#pragma unroll
+        for (int j = 0; j < kXC; ++j) {
+            write_x(0, j, xs[0][j]);
+            load_x(2, j, xs[0][j]);
         }
     }
-
-    f32x16 acc[4][4];
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb)
+    for (int slot = 0; slot < kWork0; ++slot) work0(slot, 1, kS - 1, IC<1>());
+    __syncthreads();
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb) acc[nb][mb] = (f32x16){};
-
-    // operand fragments, two sets: the reads of one k-step are issued before
-    // the 16 MFMAs of the previous one, so their LDS latency hides behind
-    // 512 cycles of matrix work instead of stalling each group of four.  F32
-    // X fragments are kept as read and rounded to BF16 next to the products
-    // that use them, so that no rounding waits on a read just issued.
-    struct XFragBf16 { vec8 b[4]; };
-    struct XFragF32 { f32x4 u[4], v[4]; };
-    typedef typename std::conditional<XF32, XFragF32, XFragBf16>::type XFrag;
-    vec8 fa0[4], fa1[4];
-    XFrag fb0, fb1;
-    auto read = [&](int st, int ks, vec8 fa[4], XFrag &fb) __attribute__((always_inline)) {
-        const lds_t *s = sbase + st * kStage;
+    for (int i = 0; i < 8; ++i) read_a(0, IC<0>(), i);
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb)
-            fa[nb] = *reinterpret_cast<const __attribute__((address_space(3))) vec8 *>(s + a_rd[ks] + nb * 32 * 64);
+    for (int j = 0; j < MB; ++j) read_b(0, IC<0>(), j);
+    // Step kt (p = kt & 1: W set, F32 X's buffer; buf = kt % kS).  Stage kt +
+    // 1 is published in the middle, when every wave's reads of stage kt have
+    // returned: what follows may overwrite its buffers.
+    int buf = 0;
+    auto step = [&](int kt, auto p_c) __attribute__((always_inline)) {
+        constexpr int p = decltype(p_c)::value;
+        const int cur = buf, prev = buf == 0 ? kS - 1 : buf - 1;
+        __builtin_amdgcn_sched_barrier(0);
+        products(p_c, IC<0>(), [&](int i) __attribute__((always_inline)) {
+            if (i % 2 == 0 && i / 2 < MB) read_b(XF32 ? p : cur, IC<1>(), i / 2);
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb) {
-            if constexpr (XF32) {
-                fb.u[mb] = *reinterpret_cast<const __attribute__((address_space(3))) f32x4 *>(s + b_rd[ks][0] + mb * 32 * 128);
-                fb.v[mb] = *reinterpret_cast<const __attribute__((address_space(3))) f32x4 *>(s + b_rd[ks][1] + mb * 32 * 128);
-            } else {
-                fb.b[mb] = *reinterpret_cast<const __attribute__((address_space(3))) vec8 *>(s + b_rd[ks][0] + mb * 32 * 64);
-            }
-        }
-    };
-    // the 16 MFMAs of one k-step; with dma, the DMAs of stage dkt (into
-    // buffer dst) spread over them, one group after every two MFMAs, so that
-    // their data does not reach the LDS in one burst that holds up the
-    // fragment reads (5-10% over issuing a stage's DMAs together)
-    auto mfmas = [&](const vec8 fa[4], const XFrag &fb, bool dma, int dkt, int dst) __attribute__((always_inline)) {
-#pragma unroll
-        for (int mb = 0; mb < 4; ++mb) {
-            vec8 b;
-            if constexpr (XF32) {
-                const f32x4 u = fb.u[mb], v = fb.v[mb];
-                const u32x4 w = {E::pack2(u.x, u.y), E::pack2(u.z, u.w), E::pack2(v.x, v.y), E::pack2(v.z, v.w)};
-                b = __builtin_bit_cast(vec8, w);
-            } else {
-                b = fb.b[mb];
-            }
-#pragma unroll
-            for (int hp = 0; hp < 2; ++hp) {
-#pragma unroll
-                for (int nb = 2 * hp; nb < 2 * hp + 2; ++nb) acc[nb][mb] = E::mfma(fa[nb], b, acc[nb][mb]);
-                __builtin_amdgcn_sched_barrier(0);
-                if (dma) {
-#pragma unroll
-                    for (int j = 0; j < kPer; ++j)
-                        if (j * 8 / kPer == 2 * mb + hp) dma_j(dkt, dst, j);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-    };
-    // a stage is complete in LDS for every wave: this wave's DMAs of it have
-    // landed (the `later` stages issued after it may be in flight; DMAs
-    // complete in issue order), then the barrier
-    auto publish = [&](int later) __attribute__((always_inline)) {
-        static_assert(3 * kPer <= 63, "vmcnt range");
-        if (later >= 3)
-            asm volatile("s_waitcnt vmcnt(%0)" :: "n"(3 * kPer) : "memory");
-        else if (later == 2)
-            asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * kPer) : "memory");
-        else if (later == 1)
-            asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kPer) : "memory");
-        else
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            for (int slot = 0; slot < kWork1; ++slot)
+                if (1 + slot * (8 * MB) / kWork1 == i) work1(slot, kt + 1, prev);
+        });
+        buf = buf == kS - 1 ? 0 : buf + 1;
+        // stage kt + 1 was issued kS - 2 whole intervals ago; loads and DMAs
+        // complete in issue order
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((kS - 2) * kVm) : "memory");
         __syncthreads();
-    };
-
-    // Step kt (stage st = kt % S): 16 MFMAs of k-step 0 while the fragments
-    // of k-step 1 load, the DMAs of stage kt+S-1 spread over them; publish
-    // stage kt+1 (its DMAs landed, later stages' may be in flight); 16 MFMAs
-    // of k-step 1 while the fragments of stage kt+1's k-step 0 load.
-    constexpr int kLead = kS - 1;
-    const int nk = a.K / kMmBK;
+        __builtin_amdgcn_sched_barrier(0);
+        products(p_c, IC<1>(), [&](int i) __attribute__((always_inline)) {
+            constexpr int kGap = MB == 4 ? 2 : 1;   // products between fragment reads
+            if (i % kGap == 0) {
+                const int r = i / kGap;
+                if (r < 8)
+                    read_a(buf, IC<1 - p>(), r);
+                else if (r < 8 + MB)
+                    read_b(XF32 ? 1 - p : buf, IC<0>(), r - 8);
+            }
 #pragma unroll
-    for (int j = 0; j < kLead; ++j)
-        if (j < nk) issue(j, j);
-    publish(min(kLead, nk) - 1);
-    read(0, 0, fa0, fb0);
-    int st = 0;
-    // The last step is peeled so that every step of the loop issues the same
-    // LDS reads (a read under a branch makes the wait counts conservative);
-    // sched_barrier keeps the compiler from moving reads next to their uses.
-    for (int kt = 0; kt + 1 < nk; ++kt) {
-        const int st1 = st == kS - 1 ? 0 : st + 1;
-        // stage kt+S-1 goes into the buffer of stage kt-1, whose reads all
-        // completed before the previous barrier (its fence drains them)
-        read(st, 1, fa1, fb1);
-        __builtin_amdgcn_sched_barrier(0);
-        mfmas(fa0, fb0, kt + kLead < nk, kt + kLead, st == 0 ? kS - 1 : st - 1);
-        __builtin_amdgcn_sched_barrier(0);
-        publish(min(kLead, nk - 1 - kt) - 1);
-        read(st1, 0, fa0, fb0);
-        __builtin_amdgcn_sched_barrier(0);
-        mfmas(fa1, fb1, false, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        st = st1;
+            for (int slot = 0; slot < kWork0; ++slot)
+                if (1 + slot * (8 * MB) / kWork0 == i) work0(slot, kt + 2, cur, p_c);
+        });
+    };
+    static_assert((kS - 2) * kVm <= 63, "vmcnt range");
+    int kt = 0;
+    for (; kt + 1 < nk; kt += 2) {
+        step(kt, IC<0>());
+        step(kt + 1, IC<1>());
     }
-    read(st, 1, fa1, fb1);
-    __builtin_amdgcn_sched_barrier(0);
-    mfmas(fa0, fb0, false, 0, 0);
-    mfmas(fa1, fb1, false, 0, 0);
-    static_assert(kPer == (XF32 ? 12 : 8), "per-stage DMA count");
+    if (kt < nk) step(kt, IC<0>());
+    // (the products are asm: the wait states between the last and a read of
+    // its accumulators are ours to give)
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15" ::: "memory");
+    __syncthreads();
 
     // ---- epilogue: dst[m][n .. n+3] = acc (+ bias) ----------------------------
-    // Through LDS, one 32-output block (128 bytes of each of the wave's 128
+    // Through LDS, one 32-output block (128 bytes of each of the wave's 32 MB
     // token rows) at a time: the lanes leave their 16-byte pieces in the
-    // wave's own 16 KiB (chunk index XOR (row >> 1) & 7: no bank conflicts),
+    // wave's own region (chunk index XOR (row >> 1) & 7: no bank conflicts),
     // then lane L reads chunk L % 8 of row 8j + L / 8, so that every store
-    // instruction writes eight whole 128-byte lines of dst instead of
-    // 32-byte pieces of 32 rows, as streaming (nontemporal) stores: dst is
-    // not read again here (1%).  The stage buffers are free once every wave
-    // is past its last read; after that a wave touches only its own region
-    // (its LDS operations complete in order).
-    __syncthreads();
-    lds_t *const sO = sbase + wave * 32768;
+    // instruction writes eight whole 128-byte lines of dst, as streaming
+    // (nontemporal) stores: dst is not read again here (1%).  A wave touches
+    // only its own region (its LDS operations complete in order).
+    lds_t *const sO = sbase + wave * 8192 * MB;
     const int rr = lane >> 3;
     const int rc = lane & 7;
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
-        lds_t *const so = sO + (nb & 1) * 16384;
+        lds_t *const so = sO + (nb & 1) * 4096 * MB;
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb) {
-            const int row = 32 * mb + l32;
+        for (int j = 0; j < 2 * MB; ++j) {
+            const int row = 16 * j + l16;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const f32x4 v = {acc[nb][mb][4 * g], acc[nb][mb][4 * g + 1], acc[nb][mb][4 * g + 2],
-                                 acc[nb][mb][4 * g + 3]};
+            for (int i = 0; i < 2; ++i)
                 *reinterpret_cast<__attribute__((address_space(3))) f32x4 *>(
-                    so + row * 128 + (((2 * g + hi) ^ ((row >> 1) & 7)) << 4)) = v;
-            }
+                    so + row * 128 + (((4 * i + q4) ^ ((row >> 1) & 7)) << 4)) = acc[2 * nb + i][j];
         }
         const int n = n0 + 128 * wn + 32 * nb + 4 * rc;
         f32x4 bias = {0.f, 0.f, 0.f, 0.f};
         if (a.bias && n < a.N) bias = *reinterpret_cast<const f32x4 *>(a.bias + n);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
+        for (int j = 0; j < 4 * MB; ++j) {
             const int row = 8 * j + rr;
             f32x4 v = *reinterpret_cast<const __attribute__((address_space(3))) f32x4 *>(
                 so + row * 128 + ((rc ^ ((row >> 1) & 7)) << 4));
-            const int m = m0 + 128 * wm + row;
+            const int m = m0 + 32 * MB * wm + row;
             if (m < a.M && n < a.N) {
                 v.x += bias.x; v.y += bias.y; v.z += bias.z; v.w += bias.w;
                 __builtin_nontemporal_store(v, reinterpret_cast<f32x4 *>(a.dst + (int64_t)m * a.d_nb1 + (int64_t)n * 4));
@@ -382,11 +380,25 @@ void mm_bf16(MmArgs a) {
     }
 }
 
-hipError_t launch_mm(const MmArgs &a, bool x_f32, hipStream_t s) {
+template <int MB>
+static void launch_mm_t(MmArgs a, bool x_f32, hipStream_t s) {
+    a.tiles_n = (a.N + kMmBN - 1) / kMmBN;
+    a.tiles_m = (a.M + 64 * MB - 1) / (64 * MB);
+    a.n_blocks = a.tiles_n * a.tiles_m;
+    // columns of 4 output tiles (of 1, 2, 16: 3-8% slower at 63,488 x 4096 x
+    // 4096), or all of up to 8
+    a.cols = a.tiles_n <= 8 ? a.tiles_n : 4;
     if (x_f32)
-        hipLaunchKernelGGL(mm_bf16<true>, dim3(a.n_blocks), dim3(64 * kMmWaves), 0, s, a);
+        hipLaunchKernelGGL((mm_bf16<true, MB>), dim3(a.n_blocks), dim3(64 * kMmWaves), 0, s, a);
     else
-        hipLaunchKernelGGL(mm_bf16<false>, dim3(a.n_blocks), dim3(64 * kMmWaves), 0, s, a);
+        hipLaunchKernelGGL((mm_bf16<false, MB>), dim3(a.n_blocks), dim3(64 * kMmWaves), 0, s, a);
+}
+
+hipError_t launch_mm(const MmArgs &a, int tile, bool x_f32, hipStream_t s) {
+    if (tile == 88)
+        launch_mm_t<4>(a, x_f32, s);
+    else
+        launch_mm_t<2>(a, x_f32, s);
     return hipGetLastError();
 }
 

@@ -1,4 +1,4 @@
-"""The few-token kernels of the linear-layer product (kd_mm_ksplit.hip)
+"""The kernels of the linear-layer product (mm_skinny, mm_ksplit, mm_bf16)
 against the float64 product of the same BF16-rounded operands: tokens at and
 past every boundary of the kernel choice and of the tiles, outputs that end
 inside a tile, k of one half stage, whole stages, a half last one and more
@@ -23,12 +23,13 @@ CASES = [(1, 4, 32), (8, 36, 96), (9, 100, 416), (16, 260, 1184), (3, 16388, 288
          (850, 2100, 672),    # 128 x 64
          (700, 4100, 352),    # 128 x 96
          (1030, 8000, 736),   # 128 x 128
-         (2049, 4064, 352)]
+         (1540, 4100, 96), (1700, 4096, 32), (2047, 4004, 352),   # 256 x 128
+         (3900, 4080, 96), (3841, 4064, 64), (4090, 4064, 416)]   # 256 x 256
 
 
 @pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
-def test_few_tokens(case, xdt):
+def test_every_tile(case, xdt):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     M, N, K = case
