@@ -130,7 +130,6 @@ hipError_t dequant(const kd_fa_tensor &w, void *out, hipStream_t s) {
     a.K = (int32_t)w.ne[0];
     a.N = (int32_t)w.ne[1];
     a.out = static_cast<char *>(out);
-    a.out_nb1 = w.ne[0] * 2;
     return kdfa::launch_dequant(a, s);
 }
 

@@ -43,8 +43,7 @@ struct DqArgs {
     int64_t w_nb1;
     int32_t type;        // KD_MM_TYPE_*
     int32_t N, K;
-    char *out;           // BF16 rows [N][K], row stride out_nb1 bytes
-    int64_t out_nb1;
+    char *out;           // BF16 rows [N][K], back to back
 };
 
 // Enqueue the expansion of a weight to BF16 rows.

@@ -3,6 +3,8 @@ against the float64 product of the same BF16-rounded operands: tokens at and
 past every boundary of the kernel choice and of the tiles, outputs that end
 inside a tile, k of one half stage, whole stages, a half last one and more
 stages than the LDS rings hold, rows with padding behind them."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -57,3 +59,37 @@ def test_every_tile(case, xdt):
     assert kd_mm.run_desc(d) == 0
     torch.cuda.synchronize()
     assert np.array_equal(out.cpu().numpy(), got.numpy())
+
+
+@pytest.mark.parametrize("shape", [(1, 32), (3, 96), (71, 352), (129, 4096)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("kind", ["q8_0", "q4_0", "bf16", "f16", "f32"])
+def test_dequant_padded_rows(kind, shape):
+    """Rows back to back and rows with padding behind them: bitwise the
+    oracle's values rounded to BF16, up to the last row and no further."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    N, K = shape
+    print(f"[case] dequant {kind} {shape}", flush=True)
+    w = (np.random.default_rng(N + K).standard_normal((N, K)) * 0.05).astype(np.float32)
+    if kind in ("q8_0", "q4_0"):
+        qt = oq.TYPE_Q8_0 if kind == "q8_0" else oq.TYPE_Q4_0
+        blocks = oq.quantize_q8_0(w) if kind == "q8_0" else oq.quantize_q4_0(w)
+        values = oq.dequantize(blocks, qt, K)
+        rows, pad = torch.from_numpy(blocks), 6
+        wrap = lambda t: kd_mm.QuantWeight(t, qt, K)
+    else:
+        rows = torch.from_numpy(w).to({"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[kind])
+        values, pad = rows.float().numpy(), 8
+        wrap = lambda t: t
+    expect = torch.from_numpy(oq.round_bf16(values)).to(torch.bfloat16)
+    wide = torch.zeros((N, rows.shape[1] + pad), dtype=rows.dtype, device=DEV)
+    wide[:, :rows.shape[1]] = rows.to(DEV)
+    for src in (rows.to(DEV), wide[:, :rows.shape[1]]):
+        weight = wrap(src)
+        out = torch.full((N * K + 8,), 7.0, dtype=torch.bfloat16, device=DEV)
+        view = kd_mm.w_view(weight)
+        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        assert kd_mm._lib().kd_mm_dequant(ctypes.byref(view), ctypes.c_void_p(out.data_ptr()), N * K * 2, stream) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(out[:N * K].cpu().view(torch.int16), expect.reshape(-1).view(torch.int16))
+        assert bool((out[N * K:] == 7.0).all())
