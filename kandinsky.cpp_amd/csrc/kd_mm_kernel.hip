@@ -157,19 +157,31 @@ hipError_t launch_dequant(const DqArgs &a, hipStream_t s) {
 // against 1,700 for 32 x 32 x 16 (register operands only; on zeros 2,440 and
 // 2,480).
 //
-// K advances 32 per stage.  W (256 rows x 64 bytes) comes by DMA
-// (global_load_lds_dwordx4), kS - 1 stages ahead; BF16 X the same way, with
-// its stage.  F32 X is loaded into registers two stages ahead of its
-// rounding to BF16 and its way into one of two LDS buffers, so that it costs
-// the LDS the same as BF16 X: read from LDS as F32, X alone kept it busy for
-// 768 of a stage's 1,024 matrix cycles.  In LDS 16-byte chunk c of row r
-// lies at c ^ ((r >> 2) & 3): the 16 rows that 16 lanes of an operand read
-// touch fill the 64 banks once.  Per stage a wave reads 8 W and 2 MB X
-// fragments and issues 16 MB MFMAs in two halves (all W against half of X),
-// the DMAs of a later stage spread over the first, the loads, roundings and
-// LDS writes of X over the second; the one barrier, between them, publishes
-// the next stage.  The loop has no conditions: past the last stage the DMAs
-// and loads bring the last one again.
+// K advances 32 per stage.  With BF16 X, W (256 rows x 64 bytes) and X come
+// by DMA (global_load_lds_dwordx4), kS - 1 stages ahead.  F32 X is loaded
+// into registers two stages ahead of its rounding to BF16 and its way into
+// one of two LDS buffers, so that it costs the LDS the same as BF16 X: read
+// from LDS as F32, X alone kept it busy for 768 of a stage's 1,024 matrix
+// cycles.  That leaves LDS for W in double stages of 64 k, whole 128-byte
+// lines of its rows: a line asked for in two halves a stage apart crosses
+// from the L2 twice (from every CU, rows of 64 bytes arrive at 65 KB per
+// microsecond and CU, of 128 at 128; 16,000 x 4096 x 16384 2.11 -> 1.85 ms).
+// In LDS 16-byte chunk c of row r lies at c ^ ((r >> 2) & 3) (of a 128-byte
+// row, at c ^ ((r >> 1) & 7)): the 16 rows that 16 lanes of an operand read
+// touch fill the 64 banks once.
+//
+// Per stage a wave reads 8 W and 2 MB X fragments and issues 16 MB MFMAs in
+// two halves (all W against half of X); the fragment reads of what follows,
+// the DMAs of a later stage and X's loads, roundings and LDS writes are
+// spread over them one by one (the reads in one burst behind the barrier:
+// 10% more at BF16 x); the one barrier, between the halves, publishes the
+// next stage.  The loop has no conditions: past the last stage the DMAs and
+// loads bring the last one again.
+//
+// 63,488 x 4096 x 4096: F32 x 2.30 -> 1.99 ms, BF16 x 1.89 -> 1.69 ms
+// against 32 x 32 x 16 products with F32 X read from LDS; 4,000 tokens, F32
+// x, 149 -> 120 us.  The large calls run at the power limit (with every load
+// taken out the products alone took 75% of the time).
 // Rows past M or N read clamped (repeated) rows and are not stored.  The
 // output goes through LDS so that its stores are whole 128-byte lines.
 // ---------------------------------------------------------------------------
@@ -184,10 +196,11 @@ void mm_bf16(MmArgs a) {
     constexpr int BM = 64 * MB;
     constexpr int kXTile = BM * 64;                        // BF16 X rows of a stage
     constexpr int kS = XF32 ? 6 : MB == 4 ? 5 : 6;         // stages of W (and BF16 X) in LDS
+    constexpr int kWRing = 4;                              // F32 X: double stages of W (128-byte rows)
         constexpr int kXC = 2 * MB;                            // F32 X: 16-byte loads of a thread per stage
     constexpr int kXD = XF32 ? 0 : MB;                     // BF16 X: DMAs of a wave per stage
     constexpr int kVm = 4 + (XF32 ? kXC : kXD);            // vector memory operations of a wave per stage
-    constexpr int kX0 = kS * kMmWTile;                     // the X buffers behind W's
+    constexpr int kX0 = XF32 ? kWRing * 2 * kMmWTile : kS * kMmWTile;   // the X buffers behind W's
     constexpr int kUse = kX0 + (XF32 ? 2 : kS) * kXTile;
     constexpr int kEpi = kMmWaves * 8192 * MB;             // two blocks of 32 outputs per wave
     __shared__ __attribute__((aligned(1024))) char lds[kUse > kEpi ? kUse : kEpi];
@@ -213,11 +226,15 @@ void mm_bf16(MmArgs a) {
     const int m0 = mt * BM;
 
     // DMA lane offsets, relative to the tile's first row
-    uint32_t w_off[4], xd_off[XF32 ? 1 : MB], x_off[kXC];
+    constexpr int kWD = XF32 ? 8 : 4;                      // W's DMAs of a wave per (double) stage
+    uint32_t w_off[kWD], xd_off[XF32 ? 1 : MB], x_off[kXC];
     const int dr = lane >> 2, dc = (lane & 3) ^ ((lane >> 4) & 3);   // chunk dc of row 16 i + dr
+    const int wc = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);      // chunk wc of row 8 i + lane / 8 (double stages)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-        w_off[j] = (uint32_t)min(16 * (wave + kMmWaves * j) + dr, a.N - 1 - n0) * (uint32_t)a.w_nb1 + (uint32_t)(dc << 4);
+    for (int j = 0; j < kWD; ++j) {
+        const int r = XF32 ? 8 * (wave + kMmWaves * j) + (lane >> 3) : 16 * (wave + kMmWaves * j) + dr;
+        w_off[j] = (uint32_t)min(r, a.N - 1 - n0) * (uint32_t)a.w_nb1 + (uint32_t)((XF32 ? wc : dc) << 4);
+    }
     if constexpr (XF32) {
         // load j of a thread: 4 F32 of row 8 (wave + 4 j) + lane / 8, to
         // x_wr + 2048 j of an X buffer
@@ -245,6 +262,14 @@ void mm_bf16(MmArgs a) {
         else if constexpr (!XF32)
             dma16(xtile + k64, xd_off[j - 4], sbase + kX0 + buf * kXTile + (wave + kMmWaves * (j - 4)) * 1024);
     };
+    const int nws = (nk + 1) >> 1;
+    // DMA j (of 8) of double stage ws into ring buffer wb; past K, in a last
+    // double stage with one half, the first half's chunks again
+    auto dma_w2 = [&](int ws, int wb, int j) __attribute__((always_inline)) {
+        const int w = min(ws, nws - 1);
+        const uint32_t back = (nk & 1) && w == nws - 1 && wc >= 4 ? 64u : 0u;
+        dma16(wtile + (int64_t)w * 128, w_off[j] - back, sbase + wb * 32768 + (wave + kMmWaves * j) * 1024);
+    };
     f32x4 xs[2][kXC];
     auto load_x = [&](int kt, int j, f32x4 &v) __attribute__((always_inline)) {
         v = *reinterpret_cast<const f32x4 *>(xtile + (int64_t)min(kt, nk - 1) * 128 + x_off[j]);
@@ -267,8 +292,13 @@ void mm_bf16(MmArgs a) {
         for (int j = 0; j < 2 * MB; ++j) acc[i][j] = (f32x4){};
     vec8 fa[2][8], fb[2][MB];
     typedef const __attribute__((address_space(3))) vec8 lds_v8;
+    const uint32_t a2_rd = (uint32_t)((128 * wn + l16) * 128 + ((q4 ^ ((l16 >> 1) & 7)) << 4));
     auto read_a = [&](int buf, auto p_c, int i) __attribute__((always_inline)) {
-        fa[decltype(p_c)::value][i] = *reinterpret_cast<lds_v8 *>(sbase + buf * kMmWTile + a_rd + i * 1024);
+        constexpr int p = decltype(p_c)::value;
+        if constexpr (XF32)   // buf: the ring buffer of the double stage; the second half's chunks are the first's ^ 4
+            fa[p][i] = *reinterpret_cast<lds_v8 *>(sbase + buf * 32768 + (a2_rd ^ (p << 6)) + i * 2048);
+        else
+            fa[p][i] = *reinterpret_cast<lds_v8 *>(sbase + buf * kMmWTile + a_rd + i * 1024);
     };
     auto read_b = [&](int buf, auto h_c, int j) __attribute__((always_inline)) {
         constexpr int h = decltype(h_c)::value;
@@ -291,11 +321,11 @@ void mm_bf16(MmArgs a) {
     // The vector memory work of a stage interval (between two barriers), in
     // two halves.  The first, while a step's second products run: stage dk's
     // F32 X rounded from registers (set and buffer dk & 1 = xp) into LDS and
-    // the registers loaded for stage dk + 2, or the first DMAs of stage
+    // the registers loaded for stage dk + 2, or the first DMAs of BF16 stage
     // dk + kS - 2 into its buffer dbuf.  The second, while the next step's
-    // first products run: W's DMAs of stage dk + kS - 2, or the rest of them.
-    // (F32 x, 63,488 tokens: X and W mixed in both halves 2.20 ms against
-    // 2.06.)
+    // first products run: half of a double stage of W, or the rest of those
+    // DMAs.  (F32 x, 63,488 tokens: X and W mixed in both halves 2.20 ms
+    // against 2.06.)
     constexpr int kWork0 = XF32 ? kXC : 2 + MB / 2, kWork1 = XF32 ? 4 : 2 + MB / 2;
     auto work0 = [&](int slot, int dk, int dbuf, auto xp_c) __attribute__((always_inline)) {
         constexpr int xp = decltype(xp_c)::value;
@@ -307,12 +337,22 @@ void mm_bf16(MmArgs a) {
         }
     };
     auto work1 = [&](int slot, int dk, int dbuf) __attribute__((always_inline)) {
-        dma_j(dk + kS - 2, dbuf, XF32 ? slot : kWork0 + slot);
+        if constexpr (XF32)
+            dma_w2(((dk - 1) >> 1) + kWRing - 1, dbuf, 4 * ((dk - 1) & 1) + slot);
+        else
+            dma_j(dk + kS - 2, dbuf, kWork0 + slot);
     };
+    if constexpr (XF32) {
 #pragma unroll
-    for (int s = 0; s < kS - 1; ++s)
+        for (int s = 0; s < kWRing - 1; ++s)
 #pragma unroll
-        for (int j = 0; j < 4 + kXD; ++j) dma_j(s, s, j);
+            for (int j = 0; j < 8; ++j) dma_w2(s, s, j);
+    } else {
+#pragma unroll
+        for (int s = 0; s < kS - 1; ++s)
+#pragma unroll
+            for (int j = 0; j < 4 + kXD; ++j) dma_j(s, s, j);
+    }
     if constexpr (XF32) {
 #pragma unroll
         for (int p = 0; p < 2; ++p)
@@ -335,13 +375,15 @@ void mm_bf16(MmArgs a) {
     for (int i = 0; i < 8; ++i) read_a(0, IC<0>(), i);
 #pragma unroll
     for (int j = 0; j < MB; ++j) read_b(0, IC<0>(), j);
-    // Step kt (p = kt & 1: W set, F32 X's buffer; buf = kt % kS).  Stage kt +
-    // 1 is published in the middle, when every wave's reads of stage kt have
+    // Step kt (p = kt & 1: W set, F32 X's buffer; buf = kt % kS, or the
+    // double stage's ring buffer, (kt / 2) % kWRing).  Stage kt + 1 is
+    // published in the middle, when every wave's reads of stage kt have
     // returned: what follows may overwrite its buffers.
     int buf = 0;
     auto step = [&](int kt, auto p_c) __attribute__((always_inline)) {
         constexpr int p = decltype(p_c)::value;
-        const int cur = buf, prev = buf == 0 ? kS - 1 : buf - 1;
+        constexpr int kRing = XF32 ? kWRing : kS;
+        const int cur = buf, prev = buf == 0 ? kRing - 1 : buf - 1;
         __builtin_amdgcn_sched_barrier(0);
         products(p_c, IC<0>(), [&](int i) __attribute__((always_inline)) {
             if (i % 2 == 0 && i / 2 < MB) read_b(XF32 ? p : cur, IC<1>(), i / 2);
@@ -349,10 +391,11 @@ void mm_bf16(MmArgs a) {
             for (int slot = 0; slot < kWork1; ++slot)
                 if (1 + slot * (8 * MB) / kWork1 == i) work1(slot, kt + 1, prev);
         });
-        buf = buf == kS - 1 ? 0 : buf + 1;
-        // stage kt + 1 was issued kS - 2 whole intervals ago; loads and DMAs
-        // complete in issue order
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((kS - 2) * kVm) : "memory");
+        if (!XF32 || p == 1) buf = buf == kRing - 1 ? 0 : buf + 1;
+        // stage kt + 1 (W's double stage kt / 2 + 1) was issued kS - 2 (2
+        // kWRing - 4) whole intervals ago; loads and DMAs complete in issue
+        // order
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((XF32 ? 2 * (kWRing - 2) : kS - 2) * kVm) : "memory");
         __syncthreads();
         __builtin_amdgcn_sched_barrier(0);
         products(p_c, IC<1>(), [&](int i) __attribute__((always_inline)) {
@@ -369,7 +412,7 @@ void mm_bf16(MmArgs a) {
                 if (1 + slot * (8 * MB) / kWork0 == i) work0(slot, kt + 2, cur, p_c);
         });
     };
-    static_assert((kS - 2) * kVm <= 63, "vmcnt range");
+    static_assert((XF32 ? 2 * (kWRing - 2) : kS - 2) * kVm <= 63, "vmcnt range");
     int kt = 0;
     for (; kt + 1 < nk; kt += 2) {
         step(kt, IC<0>());
