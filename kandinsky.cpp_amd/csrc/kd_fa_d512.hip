@@ -16,44 +16,54 @@ namespace kdfa {
 // (src/models/vae.hpp:60-101 -> ops::attention with one head, D = channels =
 // 512), no mask, no RoPE.
 //
-// A workgroup is 4 waves and covers R blocks of 32 query rows of one (b, h);
-// wave w owns the 128 columns 128w .. 128w+127 of D for both products, so
-// that its O (32R rows x 128) and Q (32R rows x 128) stay in registers.  Per
-// 32-key tile:
-//   S_w^T = K_w Q_w^T over the wave's 128 columns (8 MFMA per row block), K
-//           fragments straight from global memory (each wave reads only its
-//           columns, once for all R blocks);
+// A workgroup is 4 waves (one per CU: 119-141 KB of LDS) and covers R blocks
+// of 32 query rows of one (b, h); wave w owns the 128 columns 128w .. 128w+127
+// of D for both products, so that its O (32R rows x 128) and Q (32R rows x
+// 128) stay in registers.  Per 32-key tile:
+//   S_w^T = K_w Q_w^T over the wave's 128 columns (8 MFMA per row block), K_w
+//           staged by DMA in the wave's own LDS region (loaded straight into
+//           the operands, a lane's neighbours in other rows, K came at 38 KB
+//           per microsecond and CU against 130 by whole row pieces);
 //   the four partial scores meet in LDS; wave w runs the online softmax of
 //           rows 8Rw .. 8Rw+8R-1 (exact running max, exp2 domain) and writes
 //           the weights P (rounded to the operand type), the rescale factor
 //           and, at the end, the row sum to LDS for all waves;
-//   O_w^T = alpha * O_w^T + V_w^T P^T (8 MFMA per row block), V_w staged by
-//           DMA in the wave's own LDS region (NB buffers, no barrier: only
-//           that wave reads it) and read transposed with ds_read_b64_tr_b16,
-//           each fragment once for all R blocks.
-// NB = 2 (R = 2): V(t+1) staged during tile t, one workgroup per CU.  NB = 1
-// (R = 1, 54 KB of LDS, 228 registers): two workgroups per CU, so that one
-// hides the other's barrier and LDS round trips; V(t+1) is staged once
-// PV(t) has read V(t), and K is loaded two tiles ahead instead.
-// Two barriers per tile.  Keys past Lk (last tile) load clamped rows and get
-// weight 0.  Every K and V byte a workgroup streams serves 32R query rows:
-// with R = 2 the key stream of the long latents (16,384 keys, all of them
-// re-read by every workgroup) halves.  R = 1 and R = 2 give bitwise equal
-// results: the same products, the same sums of the partial scores, and the
-// row sums combined in the same tree (4 keys per leaf).
+//   O_w^T = alpha * O_w^T + V_w^T P^T (8 MFMA per row block), V_w staged the
+//           same way (two buffers) and read transposed with
+//           ds_read_b64_tr_b16, each fragment once for all R blocks.
+// Two barriers per tile.  Keys past Lk (last tile) come as zeros and get
+// weight 0.  Every K and V byte a workgroup streams serves 32R query rows.
+// R = 1 and R = 2 give bitwise equal results: the same products, the same
+// sums of the partial scores, and the row sums combined in the same tree (4
+// keys per leaf).
 // With a key split (a.n_split > 1, short query sets with a workspace), a
 // workgroup runs only its range of key tiles and leaves the unnormalised O,
 // running max and row sum of its rows for d512_combine.
+// What binds is LDS: at R = 2 a tile moves 212 KB through it (1,650 of its
+// about 2,900 cycles; the products take 1,024).  F16 K / V: 4,096 tokens with
+// the key split 96.8 -> 73.4 us, 8,192 311 -> 205, 16,384 924 -> 706; with
+// the products in sequence with the exchange and the DMAs in one burst
+// before the barrier 16,384 tokens took 880.
 constexpr int kD5 = 512;                     // D, four 128-column slices
 constexpr int kD5Keys = 32;                    // keys per tile
 constexpr int kD5SStride = kD5Keys + 4;        // floats per row of a partial-score block (pad)
 constexpr int kD5PStride = kD5Keys + 8;        // 16-bit weights per row of P (pad)
-constexpr int kD5VTile = kD5Keys * 256;        // one wave's V tile: 32 keys x 128 columns
+constexpr int kD5Tile = kD5Keys * 256;         // one wave's K or V tile: 32 keys x 128 columns
 
 static_assert(kD5 == 4 * 128, "one 128-column slice per wave");
 
-template <typename T, int R, int NB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 2 : 1, NB == 1 ? 2 : 1)))
+// the value of lane l ^ X within each row's lanes (X = 1, 2, 4: quad_perm
+// for the first two, row_half_mirror for the third, whose mirrored lane
+// holds the same as lane l ^ 4 once the quads agree)
+template <int X>
+static __device__ __forceinline__ float row_xor(float v) {
+    const int i = __builtin_bit_cast(int, v);
+    constexpr int kCtrl = X == 1 ? 0xB1 : X == 2 ? 0x4E : 0x141;
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, kCtrl, 0xF, 0xF, true));
+}
+
+template <typename T, int R>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void fa_fwd_d512(Args a) {
     typedef Elem<T> E;
     typedef typename E::vec8 vec8;
@@ -64,7 +74,8 @@ void fa_fwd_d512(Args a) {
     __shared__ __attribute__((aligned(16))) uint16_t sP[kRows][kD5PStride];
     __shared__ float sAlpha[kRows];
     __shared__ float sL[kRows];
-    __shared__ __attribute__((aligned(1024))) char sV[4][NB][kD5VTile];
+    __shared__ __attribute__((aligned(1024))) char sV[4][2][kD5Tile];
+    __shared__ __attribute__((aligned(1024))) char sK[4][kD5Tile];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -107,26 +118,40 @@ void fa_fwd_d512(Args a) {
 
     const char *kbase = a.k + (int64_t)(h / a.rk2) * a.k_nb2 + (int64_t)(b / a.rk3) * a.k_nb3 + col0 * 2;
     const char *vbase = a.v + (int64_t)(h / a.rv2) * a.v_nb2 + (int64_t)(b / a.rv3) * a.v_nb3 + col0 * 2;
-    // K fragment of k-step ks: key (tile row) l32, columns ks*16 + hi*8 .. +7
-    auto load_k = [&](int t, vec8 kf[8]) __attribute__((always_inline)) {
-        int key = t * kD5Keys + l32;
-        key = key < Lk ? key : Lk - 1;
-        const char *kp = kbase + (int64_t)key * a.k_nb1 + hi * 16;
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) kf[ks] = __builtin_bit_cast(vec8, ld16(kp + ks * 32));
-    };
-    // V tile of this wave: LDS row r (key t*32 + r, clamped) holds the wave's
-    // 128 columns, 16-byte chunk c at c ^ v_swz(r); 8 DMA rounds of 4 rows
+    // V tile of this wave: LDS row r (key t*32 + r) holds the wave's 128
+    // columns, 16-byte chunk c at c ^ v_swz(r); 8 DMA rounds of 4 rows
+    // K tile: the same rows, chunk c at c ^ (r & 15)
     const int dma_row = lane >> 4, dma_pc = lane & 15;
-    auto issue_v = [&](int t, int buf) __attribute__((always_inline)) {
-        lds_t *dst = LDS_PTR(char, sV[wave][buf]);
+    uint32_t k_off[kD5Keys / 4], v_off[kD5Keys / 4];
 #pragma unroll
-        for (int j = 0; j < kD5Keys / 4; ++j) {
-            const int r = 4 * j + dma_row;
-            int key = t * kD5Keys + r;
-            key = key < Lk ? key : Lk - 1;
-            dma16(vbase, (uint32_t)key * (uint32_t)a.v_nb1 + ((dma_pc ^ v_swz(r)) << 4), dst + j * 1024);
-        }
+    for (int j = 0; j < kD5Keys / 4; ++j) {
+        const int r = 4 * j + dma_row;
+        k_off[j] = (uint32_t)r * (uint32_t)a.k_nb1 + ((dma_pc ^ (r & 15)) << 4);
+        v_off[j] = (uint32_t)r * (uint32_t)a.v_nb1 + ((dma_pc ^ v_swz(r)) << 4);
+    }
+    // a tile's resource: from its first row to the end of its last key's
+    // 256 bytes; rows past that come as zeros
+    auto tile_rsrc = [&](const char *base, int64_t nb1, int t) __attribute__((always_inline)) {
+        const uint64_t p = (uint64_t)(base + (int64_t)t * kD5Keys * nb1);
+        const uint32_t rows = (uint32_t)min(kD5Keys, Lk - t * kD5Keys);
+        return (u32x4){(uint32_t)p, (uint32_t)(p >> 32) & 0xffffu, (rows - 1) * (uint32_t)nb1 + 256, 0x00020000u};
+    };
+    auto dma = [&](u32x4 rsrc, uint32_t off, lds_t *dst) __attribute__((always_inline)) {
+        const uint32_t m0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)dst);
+        asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" :: "v"(off), "s"(rsrc), "{m0}"(m0));
+    };
+    lds_t *const ks_ = LDS_PTR(char, sK[wave]);
+    // DMA j (of 8) of a tile: rows 4 j .. 4 j + 3
+    auto dma_k = [&](u32x4 rsrc, int j) __attribute__((always_inline)) { dma(rsrc, k_off[j], ks_ + j * 1024); };
+    auto dma_v = [&](u32x4 rsrc, int buf, int j) __attribute__((always_inline)) {
+        dma(rsrc, v_off[j], LDS_PTR(char, sV[wave][buf]) + j * 1024);
+    };
+    // K fragment of k-step i: key (tile row) l32, columns 16 i + 8 hi .. +7
+    auto read_k = [&](vec8 kf[8]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            kf[i] = *reinterpret_cast<const __attribute__((address_space(3))) vec8 *>(
+                ks_ + l32 * 256 + (((2 * i + hi) ^ (l32 & 15)) << 4));
     };
     const int v_sub = (lane & 15) >> 2;
     const int v_c_lo = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
@@ -146,99 +171,63 @@ void fa_fwd_d512(Args a) {
     const int skey = kKeysPerLane * (lane % kLanesPerRow);
     float m_run = -INFINITY, l_run = 0.0f;
 
-    // VMEM order per tile: the V DMA (inline asm, invisible to the
-    // compiler's vmcnt bookkeeping) before the K loads, so that the
-    // compiler's own waits for K stay exact (loads complete in order) and
-    // V(t) has landed once at most the 16 newer loads are in flight
-    // NB = 1 (one V buffer per wave, two workgroups per CU): K fragments
-    // two tiles ahead in two register sets, V(t+1) staged once PV(t) has
-    // read V(t); VMEM order K(t+2) .. V(t+1), so the compiler's wait for K
-    // never waits for the V DMA issued after it
-    vec8 kf[NB == 1 ? 2 : 1][8];
-    if (n_tiles > t_begin) {
-        if constexpr (NB == 2) {
-            issue_v(t_begin, t_begin & 1);
-            load_k(t_begin, kf[0]);
-        } else {
-            load_k(t_begin, kf[0]);
-            if (t_begin + 1 < n_tiles) load_k(t_begin + 1, kf[1]);
-            issue_v(t_begin, 0);
-        }
-    }
-    auto tile = [&](int t, auto kb_c) __attribute__((always_inline)) {
-        constexpr int kb = decltype(kb_c)::value ? 1 : 0;
+    // Step t writes the partial scores of tile t, runs the products of V(t-1)
+    // while they meet, and those of K(t+1) between the steps of tile t's
+    // softmax: a wave alone on its SIMD has nothing else to run under the
+    // exchange.  Its DMAs, K(t+2) among the first products and V(t+1) among
+    // the second, take the CU's load path about as long as the products the
+    // matrix cores; at the next step's start at most V's 8 may be in flight.
+    // K's one buffer is free once its fragments are in registers, V's two
+    // alternate; both are the wave's own (no barrier).
+    f32x16 s[R];
+    vec8 kf[8];
+    auto partial = [&](int rb, int i) __attribute__((always_inline)) {
+        s[rb] = i == 0 ? E::mfma(kf[0], qf[rb][0], (f32x16){}) : E::mfma(kf[i], qf[rb][i], s[rb]);
+    };
+    auto keep_q = [&]() __attribute__((always_inline)) {
         // the Q fragments (read by the matrix unit only) live in AGPRs, so
         // that O, S and the K fragments have the VGPRs to themselves
 #pragma unroll
         for (int rb = 0; rb < R; ++rb)
 #pragma unroll
-            for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+a"(qf[rb][ks]));
-        // ---- partial scores over this wave's columns
-        f32x16 s[R];
+            for (int i = 0; i < 8; ++i) asm volatile("" : "+a"(qf[rb][i]));
+    };
+    if (n_tiles > t_begin) {
+        const u32x4 k0 = tile_rsrc(kbase, a.k_nb1, t_begin);
 #pragma unroll
-        for (int rb = 0; rb < R; ++rb) {
-            s[rb] = (f32x16){};
+        for (int j = 0; j < 8; ++j) dma_k(k0, j);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        read_k(kf);
+        keep_q();
 #pragma unroll
-            for (int ks = 0; ks < 8; ++ks) s[rb] = E::mfma(kf[kb][ks], qf[rb][ks], s[rb]);
-        }
-        if constexpr (NB == 2) {
-            if (t + 1 < n_tiles) {
-                issue_v(t + 1, (t + 1) & 1);
-                load_k(t + 1, kf[0]);
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int rb = 0; rb < R; ++rb) partial(rb, i);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        const u32x4 k1 = tile_rsrc(kbase, a.k_nb1, min(t_begin + 1, n_tiles - 1));
+#pragma unroll
+        for (int j = 0; j < 8; ++j) dma_k(k1, j);
+        const u32x4 v0 = tile_rsrc(vbase, a.v_nb1, t_begin);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) dma_v(v0, t_begin & 1, j);
+    }
+    // O_w^T = alpha * O_w^T + V_w^T P^T of tile t
+    auto pv = [&](int t, auto between) __attribute__((always_inline)) {
+        const lds_t *vs_ = LDS_PTR(char, sV[wave][t & 1]);
+        vec8 va[2][4], pb[2][R];
+#pragma unroll
+        for (int kst = 0; kst < 2; ++kst) {
+#pragma unroll
+            for (int rb = 0; rb < R; ++rb)
+                pb[kst][rb] = *reinterpret_cast<const vec8 *>(&sP[32 * rb + l32][16 * kst + 8 * hi]);
+#pragma unroll
+            for (int dblk = 0; dblk < 4; ++dblk) {
+                const lds_t *vp = vs_ + v_rd[dblk] + 4096 * kst;
+                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(vp));
+                const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(vp + 1024));
+                va[kst][dblk] = __builtin_bit_cast(vec8, __builtin_shufflevector(lo, hi4, 0, 1, 2, 3, 4, 5, 6, 7));
             }
-        } else {
-            if (t + 2 < n_tiles) load_k(t + 2, kf[kb]);
         }
-        // element i of lane l: key 8*(i/4) + 4*hi + i%4, query l32
-#pragma unroll
-        for (int rb = 0; rb < R; ++rb)
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                *reinterpret_cast<f32x4 *>(&sS[wave][32 * rb + l32][8 * g + 4 * hi]) =
-                    (f32x4){s[rb][4 * g], s[rb][4 * g + 1], s[rb][4 * g + 2], s[rb][4 * g + 3]};
-        __syncthreads();
-        // ---- softmax of the wave's rows: 4R keys per lane
-        {
-            float sc[kKeysPerLane];
-#pragma unroll
-            for (int c = 0; c < R; ++c) {
-                f32x4 x = *reinterpret_cast<const f32x4 *>(&sS[0][srow][skey + 4 * c]);
-#pragma unroll
-                for (int w = 1; w < 4; ++w)
-                    x += *reinterpret_cast<const f32x4 *>(&sS[w][srow][skey + 4 * c]);
-                sc[4 * c] = x.x * c2; sc[4 * c + 1] = x.y * c2; sc[4 * c + 2] = x.z * c2; sc[4 * c + 3] = x.w * c2;
-            }
-#pragma unroll
-            for (int e = 0; e < kKeysPerLane; ++e)
-                if (t * kD5Keys + skey + e >= k_end) sc[e] = -INFINITY;
-            float mx = sc[0];
-#pragma unroll
-            for (int e = 1; e < kKeysPerLane; ++e) mx = __builtin_fmaxf(mx, sc[e]);
-#pragma unroll
-            for (int d = 1; d < kLanesPerRow; d <<= 1) mx = __builtin_fmaxf(mx, __shfl_xor(mx, d));
-            const float m_new = __builtin_fmaxf(m_run, mx);
-            const float alpha = m_new == m_run ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
-            m_run = m_new;
-            const float mu = m_new == -INFINITY ? 0.0f : m_new;
-            float p[kKeysPerLane];
-#pragma unroll
-            for (int e = 0; e < kKeysPerLane; ++e) p[e] = __builtin_amdgcn_exp2f(sc[e] - mu);
-            // row sum: 4-key leaves (p0 + p1) + (p2 + p3) combined pairwise,
-            // the pairs within the lane first, then across lanes
-            float ps = (p[0] + p[1]) + (p[2] + p[3]);
-            if constexpr (R == 2) ps = ps + ((p[4] + p[5]) + (p[6] + p[7]));
-#pragma unroll
-            for (int d = 1; d < kLanesPerRow; d <<= 1) ps += __shfl_xor(ps, d);
-            l_run = l_run * alpha + ps;
-#pragma unroll
-            for (int c = 0; c < R; ++c) {
-                const u32x2 w = {E::pack2(p[4 * c], p[4 * c + 1]), E::pack2(p[4 * c + 2], p[4 * c + 3])};
-                *reinterpret_cast<u32x2 *>(&sP[srow][skey + 4 * c]) = w;
-            }
-            if (lane % kLanesPerRow == 0) sAlpha[srow] = alpha;
-        }
-        __syncthreads();
-        // ---- O_w^T = alpha * O_w^T + V_w^T P^T
 #pragma unroll
         for (int rb = 0; rb < R; ++rb) {
             const float al = sAlpha[32 * rb + l32];
@@ -249,44 +238,107 @@ void fa_fwd_d512(Args a) {
                     for (int i = 0; i < 16; ++i) o[rb][dblk][i] *= al;
             }
         }
-        if constexpr (NB == 2) {
-            if (t + 1 < n_tiles)
-                asm volatile("s_waitcnt vmcnt(16)" ::: "memory");   // V(t) landed; V(t+1), K(t+1) may fly
-            else
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        } else {
-            if (t + 2 < n_tiles)
-                asm volatile("s_waitcnt vmcnt(8)" ::: "memory");    // V(t) landed; K(t+2) may fly
-            else
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        }
-        const lds_t *vs_ = LDS_PTR(char, sV[wave][NB == 2 ? (t & 1) : 0]);
 #pragma unroll
-        for (int kst = 0; kst < kD5Keys / 16; ++kst) {
-            vec8 pb[R];
+        for (int kst = 0; kst < 2; ++kst)
 #pragma unroll
-            for (int rb = 0; rb < R; ++rb) pb[rb] = *reinterpret_cast<const vec8 *>(&sP[32 * rb + l32][16 * kst + 8 * hi]);
+            for (int dblk = 0; dblk < 4; ++dblk)
 #pragma unroll
-            for (int dblk = 0; dblk < 4; ++dblk) {
-                const lds_t *vp = vs_ + v_rd[dblk] + 4096 * kst;
-                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(vp));
-                const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(vp + 1024));
-                const vec8 va = __builtin_bit_cast(vec8, __builtin_shufflevector(lo, hi4, 0, 1, 2, 3, 4, 5, 6, 7));
-#pragma unroll
-                for (int rb = 0; rb < R; ++rb) o[rb][dblk] = E::mfma(va, pb[rb], o[rb][dblk]);
-            }
-        }
-        if constexpr (NB == 1) {
-            if (t + 1 < n_tiles) {
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's V(t) reads are done
-                issue_v(t + 1, 0);
-            }
-        }
+                for (int rb = 0; rb < R; ++rb) {
+                    o[rb][dblk] = E::mfma(va[kst][dblk], pb[kst][rb], o[rb][dblk]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (rb == R - 1) between(4 * kst + dblk);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
     };
-    for (int t = t_begin; t < n_tiles; t += NB == 1 ? 2 : 1) {
-        tile(t, BC<false>());
-        if constexpr (NB == 1)
-            if (t + 1 < n_tiles) tile(t + 1, BC<true>());
+    for (int t = t_begin; t < n_tiles; ++t) {
+        // ---- this wave's partial scores of tile t; element i of lane l: key
+        // 8*(i/4) + 4*hi + i%4, query l32
+#pragma unroll
+        for (int rb = 0; rb < R; ++rb)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *reinterpret_cast<f32x4 *>(&sS[wave][32 * rb + l32][8 * g + 4 * hi]) =
+                    (f32x4){s[rb][4 * g], s[rb][4 * g + 1], s[rb][4 * g + 2], s[rb][4 * g + 3]};
+        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // K(t+1) and V(t-1) have landed
+        read_k(kf);                                        // (past the last tile: the last one's, unused)
+        // K(t+2)'s DMAs (past the last tile, that one again) between the
+        // products of V(t-1): those wait for reads later than K(t+1)'s
+        const u32x4 k2 = tile_rsrc(kbase, a.k_nb1, min(t + 2, n_tiles - 1));
+        if (t > t_begin) {
+            pv(t - 1, [&](int j) __attribute__((always_inline)) { dma_k(k2, j); });
+        } else {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int j = 0; j < 8; ++j) dma_k(k2, j);
+        }
+        const u32x4 v1 = tile_rsrc(vbase, a.v_nb1, min(t + 1, n_tiles - 1));
+        __syncthreads();
+        // ---- softmax of the wave's rows (4R keys per lane)
+        f32x4 x[R][4];
+#pragma unroll
+        for (int c = 0; c < R; ++c)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) x[c][w] = *reinterpret_cast<const f32x4 *>(&sS[w][srow][skey + 4 * c]);
+        keep_q();
+        constexpr int kM = 8 * R;
+        auto mm = [&](auto from_c, auto to_c) __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = decltype(from_c)::value; i < decltype(to_c)::value; ++i) {
+                partial(i % R, i / R);
+                __builtin_amdgcn_sched_barrier(0);
+                if (i % R == R - 1) dma_v(v1, (t + 1) & 1, i / R);   // V(t-1) is read
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        mm(IC<0>(), IC<kM / 4>());   // while the partial scores arrive
+        float sc[kKeysPerLane];
+#pragma unroll
+        for (int c = 0; c < R; ++c) {
+            const f32x4 sum = ((x[c][0] + x[c][1]) + x[c][2]) + x[c][3];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sc[4 * c + e] = sum[e] * c2;
+        }
+        if (t * kD5Keys + kD5Keys > k_end) {
+#pragma unroll
+            for (int e = 0; e < kKeysPerLane; ++e)
+                if (t * kD5Keys + skey + e >= k_end) sc[e] = -INFINITY;
+        }
+        float mx = sc[0];
+#pragma unroll
+        for (int e = 1; e < kKeysPerLane; ++e) mx = __builtin_fmaxf(mx, sc[e]);
+        mx = __builtin_fmaxf(mx, row_xor<1>(mx));
+        mx = __builtin_fmaxf(mx, row_xor<2>(mx));
+        if constexpr (R == 1) mx = __builtin_fmaxf(mx, row_xor<4>(mx));
+        const float m_new = __builtin_fmaxf(m_run, mx);
+        mm(IC<kM / 4>(), IC<kM / 2>());
+        const float alpha = m_new == m_run ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+        m_run = m_new;
+        const float mu = m_new == -INFINITY ? 0.0f : m_new;
+        float p[kKeysPerLane];
+#pragma unroll
+        for (int e = 0; e < kKeysPerLane; ++e) p[e] = __builtin_amdgcn_exp2f(sc[e] - mu);
+        mm(IC<kM / 2>(), IC<3 * kM / 4>());
+#pragma unroll
+        for (int c = 0; c < R; ++c) {
+            const u32x2 w = {E::pack2(p[4 * c], p[4 * c + 1]), E::pack2(p[4 * c + 2], p[4 * c + 3])};
+            *reinterpret_cast<u32x2 *>(&sP[srow][skey + 4 * c]) = w;
+        }
+        if (lane % kLanesPerRow == 0) sAlpha[srow] = alpha;
+        mm(IC<3 * kM / 4>(), IC<kM>());
+        // row sum: 4-key leaves (p0 + p1) + (p2 + p3) combined pairwise,
+        // the pairs within the lane first, then across lanes
+        float ps = (p[0] + p[1]) + (p[2] + p[3]);
+        if constexpr (R == 2) ps = ps + ((p[4] + p[5]) + (p[6] + p[7]));
+        ps += row_xor<1>(ps);
+        ps += row_xor<2>(ps);
+        if constexpr (R == 1) ps += row_xor<4>(ps);
+        l_run = l_run * alpha + ps;
+        __syncthreads();
+    }
+    if (n_tiles > t_begin) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        pv(n_tiles - 1, [](int) {});
     }
     if (a.n_split > 1) {
         // this range's unnormalised O (times exactly 1), running max and row
@@ -354,10 +406,10 @@ __global__ __launch_bounds__(256) void d512_combine(Args a) {
     }
 }
 
-template <typename T, int R, int NB>
+template <typename T, int R>
 static hipError_t launch_d512_t(const Args &a, hipStream_t s) {
     const int64_t grid = (int64_t)a.n_blocks * (a.n_split > 1 ? a.n_split : 1);
-    hipLaunchKernelGGL((fa_fwd_d512<T, R, NB>), dim3((unsigned)grid), dim3(256), 0, s, a);
+    hipLaunchKernelGGL((fa_fwd_d512<T, R>), dim3((unsigned)grid), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
@@ -367,14 +419,10 @@ hipError_t launch_d512_combine(const Args &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// 64-row workgroups (R = 2): one per CU, V double-buffered; 32-row ones
-// (R = 1): two per CU, one V buffer per wave (4,096 tokens with the key
-// split 0.115 -> 0.106 ms, without 0.188 -> 0.181; 1,024 tokens 0.053 ->
-// 0.050; the same bits)
 hipError_t launch_d512(const Args &a, int kv_type, int rows, hipStream_t stream) {
     if (rows == 64)
-        return kv_type == KD_FA_TYPE_BF16 ? launch_d512_t<__bf16, 2, 2>(a, stream) : launch_d512_t<_Float16, 2, 2>(a, stream);
-    return kv_type == KD_FA_TYPE_BF16 ? launch_d512_t<__bf16, 1, 1>(a, stream) : launch_d512_t<_Float16, 1, 1>(a, stream);
+        return kv_type == KD_FA_TYPE_BF16 ? launch_d512_t<__bf16, 2>(a, stream) : launch_d512_t<_Float16, 2>(a, stream);
+    return kv_type == KD_FA_TYPE_BF16 ? launch_d512_t<__bf16, 1>(a, stream) : launch_d512_t<_Float16, 1>(a, stream);
 }
 
 }  // namespace kdfa

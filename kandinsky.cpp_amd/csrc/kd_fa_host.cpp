@@ -169,7 +169,7 @@ int device_ok() {
 size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
 // Key split of the D = 512 kernel through the workspace (kd_fa_run_ws):
-// when its 32-row workgroups (two per CU) would leave CUs idle (fewer than
+// when its 32-row blocks are few (fewer than
 // 512: the VAE's 64x64 latent, 4,096 tokens, gives 128) and there are at least four key
 // tiles (at two, 9.1 against 11.5 us), each row block's keys are cut into
 // S ranges of whole 32-key tiles (S <= 8, one workgroup per range), whose
@@ -180,7 +180,7 @@ struct D512Split {
     int keys = 0;
     size_t bytes = 0;
 };
-constexpr int64_t kD512Slots = 512;   // 32-row workgroups resident at once: two per CU
+constexpr int64_t kD512Slots = 512;   // 32-row blocks times ranges: one round of 64-row workgroups, one per CU
 D512Split d512_split(int64_t Lq, int64_t Lk, int64_t H, int64_t B, int route) {
     D512Split r;
     const int64_t nb32 = (Lq + 31) / 32 * H * B;
@@ -608,16 +608,20 @@ int run(const kd_fa_desc *d, const kd_fa_rope *r, const kd_fa_qk_norm *n, void *
     }
     hipStream_t hs = static_cast<hipStream_t>(stream);
     if (d->q.ne[0] == kHeadDimVae) {
-        // 64 query rows per workgroup (half the key stream per row) when that
-        // still gives every CU a workgroup, else 32; KD_FA_ROUTE_D512_R1
-        // forces 32 (for comparisons)
-        const int rows = ((route & KD_FA_ROUTE_D512_R1) || (Lq + 63) / 64 * H * B < 256) ? 32 : 64;
-        a.n_qt = (int32_t)((Lq + rows - 1) / rows);
-        a.n_blocks = (int32_t)(a.n_qt * H * B);
         // with a workspace, the key split of short query sets (the partial
         // results, then the merge into dst)
-        const D512Split sp = rows == 32 ? d512_split(Lq, a.Lk, H, B, route) : D512Split{};
-        if (sp.S > 1 && ws && ws_bytes >= sp.bytes) {
+        const D512Split sp = d512_split(Lq, a.Lk, H, B, route);
+        const bool split = sp.S > 1 && ws && ws_bytes >= sp.bytes;
+        // 64 query rows per workgroup (half the key stream per row, 1.7 times
+        // the time per tile) where that saves a round of workgroups, one per
+        // CU, else 32; KD_FA_ROUTE_D512_R1 forces 32 (for comparisons)
+        const int64_t ranges = split ? sp.S : 1;
+        const int64_t r64 = ((Lq + 63) / 64 * H * B * ranges + 255) / 256;
+        const int64_t r32 = ((Lq + 31) / 32 * H * B * ranges + 255) / 256;
+        const int rows = ((route & KD_FA_ROUTE_D512_R1) || 17 * r64 > 10 * r32) ? 32 : 64;
+        a.n_qt = (int32_t)((Lq + rows - 1) / rows);
+        a.n_blocks = (int32_t)(a.n_qt * H * B);
+        if (split) {
             a.part = static_cast<float *>(ws);
             a.n_split = sp.S;
             a.split_keys = sp.keys;
