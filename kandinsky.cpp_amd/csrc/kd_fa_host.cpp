@@ -612,13 +612,13 @@ int run(const kd_fa_desc *d, const kd_fa_rope *r, const kd_fa_qk_norm *n, void *
         // results, then the merge into dst)
         const D512Split sp = d512_split(Lq, a.Lk, H, B, route);
         const bool split = sp.S > 1 && ws && ws_bytes >= sp.bytes;
-        // 64 query rows per workgroup (half the key stream per row, 1.7 times
-        // the time per tile) where that saves a round of workgroups, one per
+        // 64 query rows per workgroup (half the key stream per row, 1.5-1.7
+        // times the time) where that saves a round of workgroups, one per
         // CU, else 32; KD_FA_ROUTE_D512_R1 forces 32 (for comparisons)
         const int64_t ranges = split ? sp.S : 1;
         const int64_t r64 = ((Lq + 63) / 64 * H * B * ranges + 255) / 256;
         const int64_t r32 = ((Lq + 31) / 32 * H * B * ranges + 255) / 256;
-        const int rows = ((route & KD_FA_ROUTE_D512_R1) || 17 * r64 > 10 * r32) ? 32 : 64;
+        const int rows = ((route & KD_FA_ROUTE_D512_R1) || 3 * r64 > 2 * r32) ? 32 : 64;
         a.n_qt = (int32_t)((Lq + rows - 1) / rows);
         a.n_blocks = (int32_t)(a.n_qt * H * B);
         if (split) {

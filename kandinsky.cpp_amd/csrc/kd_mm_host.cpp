@@ -102,21 +102,23 @@ size_t ws_bytes(const kd_mm_desc *d) {
 
 // The tile of a call (32 * (tile / 10) outputs x 32 * (tile % 10) tokens) of
 // more than kMmSkinnyRows tokens: the one whose rounds of workgroups (256 at
-// once, one per CU) take least time.  `us` is a round's time with every CU at
-// it, K = 4096 and F32 x (all scale with K, and by 0.7-0.9 with BF16 x, so
-// their order holds): small tiles move more bytes per product, large ones
-// leave CUs idle.
-int choose_tile(int64_t M, int64_t N) {
-    constexpr struct { int tile, n, m; double us; } kTiles[] = {
-        {88, 256, 256, 122.0}, {84, 256, 128, 76.0}, {44, 128, 128, 43.0}, {43, 128, 96, 36.0},
-        {42, 128, 64, 27.5},   {23, 64, 96, 27.0},   {22, 64, 64, 19.0},   {21, 64, 32, 12.5},
-        {11, 32, 32, 9.0}};
+// once, one per CU) take least time.  A round's time with every CU at it, F32
+// x, is `fixed` (first loads, sums and stores) + `us` * K / 4096; with BF16 x
+// all take 0.7-0.9 of that, so their order holds.  Small tiles move more
+// bytes per product, large ones leave CUs idle.  (Without the fixed part
+// calls of few k and many tiles took too small a tile: 5,000 x 4096 x 32
+// 36 us against 28.)
+int choose_tile(int64_t M, int64_t N, int64_t K) {
+    constexpr struct { int tile, n, m; double fixed, us; } kTiles[] = {
+        {88, 256, 256, 12.0, 110.0}, {84, 256, 128, 7.0, 69.0}, {44, 128, 128, 6.0, 37.0},
+        {43, 128, 96, 5.0, 31.0},    {42, 128, 64, 4.0, 23.5},  {23, 64, 96, 3.5, 23.5},
+        {22, 64, 64, 2.5, 16.5},     {21, 64, 32, 1.7, 10.8},   {11, 32, 32, 1.2, 7.8}};
     int best = 88;
     double least = 1e300;
     for (const auto &t : kTiles) {
         const int64_t tiles = ((N + t.n - 1) / t.n) * ((M + t.m - 1) / t.m);
         if (t.tile != 88 && tiles > kdfa::kMmMaxBlocks) continue;
-        const double cost = (double)((tiles + 255) / 256) * t.us;
+        const double cost = (double)((tiles + 255) / 256) * (t.fixed + t.us * (double)K / 4096.0);
         if (cost < least) { least = cost; best = t.tile; }
     }
     return best;
@@ -197,7 +199,7 @@ int kd_mm_run(const kd_mm_desc *desc, void *workspace, size_t workspace_bytes, v
     if (M <= kdfa::kMmSkinnyRows && N <= 32 * kdfa::kMmMaxBlocks) {
         e = kdfa::launch_mm_skinny(a, x_f32, hs);
     } else {
-        const int tile = choose_tile(M, N);
+        const int tile = choose_tile(M, N, K);
         e = tile == 88 || tile == 84 ? kdfa::launch_mm(a, tile, x_f32, hs) : kdfa::launch_mm_ksplit(a, tile, x_f32, hs);
     }
     return e == hipSuccess ? KD_FA_OK : KD_FA_ERR_LAUNCH;
