@@ -184,6 +184,13 @@ void fa_fwd_d512(Args a) {
     auto partial = [&](int rb, int i) __attribute__((always_inline)) {
         s[rb] = i == 0 ? E::mfma(kf[0], qf[rb][0], (f32x16){}) : E::mfma(kf[i], qf[rb][i], s[rb]);
     };
+    // K's fragments are in registers: what follows may overwrite its buffer.
+    // The DMAs are asm, so that nothing else makes the compiler keep them
+    // behind those reads; it adds a wait only where one may be in flight
+    auto hold_k = [&]() __attribute__((always_inline)) {
+        asm volatile("; K fragments held" ::"v"(kf[0]), "v"(kf[1]), "v"(kf[2]), "v"(kf[3]), "v"(kf[4]), "v"(kf[5]),
+                     "v"(kf[6]), "v"(kf[7]) : "memory");
+    };
     auto keep_q = [&]() __attribute__((always_inline)) {
         // the Q fragments (read by the matrix unit only) live in AGPRs, so
         // that O, S and the K fragments have the VGPRs to themselves
@@ -203,7 +210,7 @@ void fa_fwd_d512(Args a) {
         for (int i = 0; i < 8; ++i)
 #pragma unroll
             for (int rb = 0; rb < R; ++rb) partial(rb, i);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        hold_k();
         const u32x4 k1 = tile_rsrc(kbase, a.k_nb1, min(t_begin + 1, n_tiles - 1));
 #pragma unroll
         for (int j = 0; j < 8; ++j) dma_k(k1, j);
@@ -262,12 +269,17 @@ void fa_fwd_d512(Args a) {
         asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // K(t+1) and V(t-1) have landed
         read_k(kf);                                        // (past the last tile: the last one's, unused)
         // K(t+2)'s DMAs (past the last tile, that one again) between the
-        // products of V(t-1): those wait for reads later than K(t+1)'s
+        // products of V(t-1), whose operands are read after K(t+1)'s
+        // fragments: no wait of their own for those (an LDS wait for them
+        // here, ahead of V's reads, would show)
         const u32x4 k2 = tile_rsrc(kbase, a.k_nb1, min(t + 2, n_tiles - 1));
         if (t > t_begin) {
-            pv(t - 1, [&](int j) __attribute__((always_inline)) { dma_k(k2, j); });
+            pv(t - 1, [&](int j) __attribute__((always_inline)) {
+                if (j == 0) hold_k();
+                dma_k(k2, j);
+            });
         } else {
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            hold_k();
 #pragma unroll
             for (int j = 0; j < 8; ++j) dma_k(k2, j);
         }
