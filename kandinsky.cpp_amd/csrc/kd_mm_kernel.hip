@@ -420,8 +420,13 @@ void mm_bf16(MmArgs a) {
     }
     if (kt < nk) step(kt, IC<0>());
     // (the products are asm: the wait states between the last and a read of
-    // its accumulators are ours to give)
+    // its accumulators are ours to give, and the accumulators pass through
+    // what follows the wait, so that no read of them can stand before it)
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 2 * MB; ++j) asm volatile("; accumulator complete" : "+a"(acc[i][j]));
     __syncthreads();
 
     // ---- epilogue: dst[m][n .. n+3] = acc (+ bias) ----------------------------
