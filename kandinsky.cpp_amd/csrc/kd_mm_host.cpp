@@ -192,15 +192,25 @@ int kd_mm_run(const kd_mm_desc *desc, void *workspace, size_t workspace_bytes, v
     a.M = (int32_t)M;
     a.N = (int32_t)N;
     a.K = (int32_t)K;
-    if (((M + kdfa::kMmBM - 1) / kdfa::kMmBM) * ((N + kdfa::kMmBN - 1) / kdfa::kMmBN) > kI32Max) return KD_FA_ERR_SHAPE;
     a.tiles_m = a.tiles_n = a.n_blocks = a.cols = 0;
     const bool x_f32 = desc->x.type == KD_MM_TYPE_F32;
     hipError_t e;
     if (M <= kdfa::kMmSkinnyRows && N <= 32 * kdfa::kMmMaxBlocks) {
         e = kdfa::launch_mm_skinny(a, x_f32, hs);
     } else {
+        // (counted in 64 bits: M and N may be within a tile of 2^31)
         const int tile = choose_tile(M, N, K);
-        e = tile == 88 || tile == 84 ? kdfa::launch_mm(a, tile, x_f32, hs) : kdfa::launch_mm_ksplit(a, tile, x_f32, hs);
+        const int64_t tiles_n = (N + 32 * (tile / 10) - 1) / (32 * (tile / 10));
+        const int64_t tiles_m = (M + 32 * (tile % 10) - 1) / (32 * (tile % 10));
+        if (tiles_n * tiles_m > kI32Max) return KD_FA_ERR_SHAPE;
+        a.tiles_n = (int32_t)tiles_n;
+        a.tiles_m = (int32_t)tiles_m;
+        a.n_blocks = (int32_t)(tiles_n * tiles_m);
+        const bool big = tile == 88 || tile == 84;
+        // columns of 4 output tiles (of 1, 2, 16: 3-8% slower at 63,488 x
+        // 4096 x 4096), or with the large tiles all of up to 8
+        a.cols = big && tiles_n <= 8 ? a.tiles_n : 4;
+        e = big ? kdfa::launch_mm(a, tile, x_f32, hs) : kdfa::launch_mm_ksplit(a, tile, x_f32, hs);
     }
     return e == hipSuccess ? KD_FA_OK : KD_FA_ERR_LAUNCH;
 }

@@ -21,8 +21,8 @@ struct MmArgs {
     char *dst;           // F32 rows [M][N], row stride d_nb1 bytes
     int64_t w_nb1, x_nb1, d_nb1;
     int32_t M, N, K;
-    // set by the launchers: the tiles, and the output tiles per column of
-    // their order
+    // the tiles, and the output tiles per column of their order (not used by
+    // mm_skinny)
     int32_t tiles_m, tiles_n, n_blocks, cols;
 };
 

@@ -469,13 +469,7 @@ void mm_bf16(MmArgs a) {
 }
 
 template <int MB>
-static void launch_mm_t(MmArgs a, bool x_f32, hipStream_t s) {
-    a.tiles_n = (a.N + kMmBN - 1) / kMmBN;
-    a.tiles_m = (a.M + 64 * MB - 1) / (64 * MB);
-    a.n_blocks = a.tiles_n * a.tiles_m;
-    // columns of 4 output tiles (of 1, 2, 16: 3-8% slower at 63,488 x 4096 x
-    // 4096), or all of up to 8
-    a.cols = a.tiles_n <= 8 ? a.tiles_n : 4;
+static void launch_mm_t(const MmArgs &a, bool x_f32, hipStream_t s) {
     if (x_f32)
         hipLaunchKernelGGL((mm_bf16<true, MB>), dim3(a.n_blocks), dim3(64 * kMmWaves), 0, s, a);
     else

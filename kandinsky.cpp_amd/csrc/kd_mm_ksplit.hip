@@ -394,11 +394,7 @@ hipError_t launch_mm_skinny(const MmArgs &a, bool x_f32, hipStream_t s) {
 }
 
 template <int NB, int MB>
-static void launch_ksplit_t(MmArgs a, bool x_f32, hipStream_t s) {
-    a.tiles_n = (a.N + 32 * NB - 1) / (32 * NB);
-    a.tiles_m = (a.M + 32 * MB - 1) / (32 * MB);
-    a.n_blocks = a.tiles_n * a.tiles_m;
-    a.cols = 4;
+static void launch_ksplit_t(const MmArgs &a, bool x_f32, hipStream_t s) {
     if (x_f32)
         hipLaunchKernelGGL((mm_ksplit<NB, MB, true>), dim3(a.n_blocks), dim3(256), 0, s, a);
     else
