@@ -254,25 +254,31 @@ void mm_bf16(MmArgs a) {
     const char *const wtile = a.w + (int64_t)n0 * a.w_nb1;
     const char *const xtile = a.x + (int64_t)m0 * a.x_nb1;
     const int nk = a.K / kMmBK;
+    // What a DMA or load of a stage past the last one brings, where one may
+    // be (end): the tile's first chunk for every lane (not used), so that the
+    // operations in flight stay as many, but not the traffic.
     // DMA j of stage kt (W's four, then BF16 X's) into buffer buf
-    auto dma_j = [&](int kt, int buf, int j) __attribute__((always_inline)) {
-        const int64_t k64 = (int64_t)min(kt, nk - 1) * 64;
+    auto dma_j = [&](int kt, int buf, int j, auto end_c) __attribute__((always_inline)) {
+        const bool past = decltype(end_c)::value && kt >= nk;
+        const int64_t k64 = past ? 0 : (int64_t)kt * 64;
         if (j < 4)
-            dma16(wtile + k64, w_off[j], sbase + buf * kMmWTile + (wave + kMmWaves * j) * 1024);
+            dma16(wtile + k64, past ? 0 : w_off[j], sbase + buf * kMmWTile + (wave + kMmWaves * j) * 1024);
         else if constexpr (!XF32)
-            dma16(xtile + k64, xd_off[j - 4], sbase + kX0 + buf * kXTile + (wave + kMmWaves * (j - 4)) * 1024);
+            dma16(xtile + k64, past ? 0 : xd_off[j - 4], sbase + kX0 + buf * kXTile + (wave + kMmWaves * (j - 4)) * 1024);
     };
     const int nws = (nk + 1) >> 1;
     // DMA j (of 8) of double stage ws into ring buffer wb; past K, in a last
     // double stage with one half, the first half's chunks again
-    auto dma_w2 = [&](int ws, int wb, int j) __attribute__((always_inline)) {
-        const int w = min(ws, nws - 1);
-        const uint32_t back = (nk & 1) && w == nws - 1 && wc >= 4 ? 64u : 0u;
-        dma16(wtile + (int64_t)w * 128, w_off[j] - back, sbase + wb * 32768 + (wave + kMmWaves * j) * 1024);
+    auto dma_w2 = [&](int ws, int wb, int j, auto end_c) __attribute__((always_inline)) {
+        const bool past = decltype(end_c)::value && ws >= nws;
+        const uint32_t back = (nk & 1) && ws == nws - 1 && wc >= 4 ? 64u : 0u;
+        dma16(wtile + (past ? 0 : (int64_t)ws * 128), past ? 0 : w_off[j] - back,
+              sbase + wb * 32768 + (wave + kMmWaves * j) * 1024);
     };
     f32x4 xs[2][kXC];
-    auto load_x = [&](int kt, int j, f32x4 &v) __attribute__((always_inline)) {
-        v = *reinterpret_cast<const f32x4 *>(xtile + (int64_t)min(kt, nk - 1) * 128 + x_off[j]);
+    auto load_x = [&](int kt, int j, f32x4 &v, auto end_c) __attribute__((always_inline)) {
+        const bool past = decltype(end_c)::value && kt >= nk;
+        v = *reinterpret_cast<const f32x4 *>(xtile + (past ? 0 : (int64_t)kt * 128) + (past ? 0 : x_off[j]));
     };
     auto write_x = [&](int buf, int j, const f32x4 &v) __attribute__((always_inline)) {
         *reinterpret_cast<__attribute__((address_space(3))) u32x2 *>(sbase + x_wr + j * 2048 + buf * kXTile) =
@@ -327,37 +333,40 @@ void mm_bf16(MmArgs a) {
     // DMAs.  (F32 x, 63,488 tokens: X and W mixed in both halves 2.20 ms
     // against 2.06.)
     constexpr int kWork0 = XF32 ? kXC : 2 + MB / 2, kWork1 = XF32 ? 4 : 2 + MB / 2;
-    auto work0 = [&](int slot, int dk, int dbuf, auto xp_c) __attribute__((always_inline)) {
+    auto work0 = [&](int slot, int dk, int dbuf, auto xp_c, auto end_c) __attribute__((always_inline)) {
         constexpr int xp = decltype(xp_c)::value;
         if constexpr (XF32) {
             write_x(xp, slot, xs[xp][slot]);
-            load_x(dk + 2, slot, xs[xp][slot]);
+            load_x(dk + 2, slot, xs[xp][slot], end_c);
         } else {
-            dma_j(dk + kS - 2, dbuf, slot);
+            dma_j(dk + kS - 2, dbuf, slot, end_c);
         }
     };
-    auto work1 = [&](int slot, int dk, int dbuf) __attribute__((always_inline)) {
+    auto work1 = [&](int slot, int dk, int dbuf, auto end_c) __attribute__((always_inline)) {
         if constexpr (XF32)
-            dma_w2(((dk - 1) >> 1) + kWRing - 1, dbuf, 4 * ((dk - 1) & 1) + slot);
+            dma_w2(((dk - 1) >> 1) + kWRing - 1, dbuf, 4 * ((dk - 1) & 1) + slot, end_c);
         else
-            dma_j(dk + kS - 2, dbuf, kWork0 + slot);
+            dma_j(dk + kS - 2, dbuf, kWork0 + slot, end_c);
     };
+    // (as many stages as there are: with two, four took 5% of the call)
     if constexpr (XF32) {
 #pragma unroll
         for (int s = 0; s < kWRing - 1; ++s)
+            if (s < nws) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) dma_w2(s, s, j);
-    } else {
-#pragma unroll
-        for (int s = 0; s < kS - 1; ++s)
-#pragma unroll
-            for (int j = 0; j < 4 + kXD; ++j) dma_j(s, s, j);
-    }
-    if constexpr (XF32) {
+                for (int j = 0; j < 8; ++j) dma_w2(s, s, j, BC<false>());
+            }
 #pragma unroll
         for (int p = 0; p < 2; ++p)
 #pragma unroll
-            for (int j = 0; j < kXC; ++j) load_x(p, j, xs[p][j]);
+            for (int j = 0; j < kXC; ++j) load_x(p, j, xs[p][j], BC<true>());
+    } else {
+#pragma unroll
+        for (int s = 0; s < kS - 1; ++s)
+            if (s < nk) {
+#pragma unroll
+                for (int j = 0; j < 4 + kXD; ++j) dma_j(s, s, j, BC<false>());
+            }
     }
     // every stage issued so far has landed: the loop's first waits count on it
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -365,11 +374,11 @@ void mm_bf16(MmArgs a) {
 #pragma unroll
         for (int j = 0; j < kXC; ++j) {
             write_x(0, j, xs[0][j]);
-            load_x(2, j, xs[0][j]);
+            load_x(2, j, xs[0][j], BC<true>());
         }
     }
 #pragma unroll
-    for (int slot = 0; slot < kWork0; ++slot) work0(slot, 1, kS - 1, IC<1>());
+    for (int slot = 0; slot < kWork0; ++slot) work0(slot, 1, kS - 1, IC<1>(), BC<true>());
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 8; ++i) read_a(0, IC<0>(), i);
@@ -380,7 +389,7 @@ void mm_bf16(MmArgs a) {
     // published in the middle, when every wave's reads of stage kt have
     // returned: what follows may overwrite its buffers.
     int buf = 0;
-    auto step = [&](int kt, auto p_c) __attribute__((always_inline)) {
+    auto step = [&](int kt, auto p_c, auto end_c) __attribute__((always_inline)) {
         constexpr int p = decltype(p_c)::value;
         constexpr int kRing = XF32 ? kWRing : kS;
         const int cur = buf, prev = buf == 0 ? kRing - 1 : buf - 1;
@@ -389,7 +398,7 @@ void mm_bf16(MmArgs a) {
             if (i % 2 == 0 && i / 2 < MB) read_b(XF32 ? p : cur, IC<1>(), i / 2);
 #pragma unroll
             for (int slot = 0; slot < kWork1; ++slot)
-                if (1 + slot * (8 * MB) / kWork1 == i) work1(slot, kt + 1, prev);
+                if (1 + slot * (8 * MB) / kWork1 == i) work1(slot, kt + 1, prev, end_c);
         });
         if (!XF32 || p == 1) buf = buf == kRing - 1 ? 0 : buf + 1;
         // stage kt + 1 (W's double stage kt / 2 + 1) was issued kS - 2 (2
@@ -409,16 +418,21 @@ void mm_bf16(MmArgs a) {
             }
 #pragma unroll
             for (int slot = 0; slot < kWork0; ++slot)
-                if (1 + slot * (8 * MB) / kWork0 == i) work0(slot, kt + 2, cur, p_c);
+                if (1 + slot * (8 * MB) / kWork0 == i) work0(slot, kt + 2, cur, p_c, end_c);
         });
     };
     static_assert((XF32 ? 2 * (kWRing - 2) : kS - 2) * kVm <= 63, "vmcnt range");
+    // the loop's steps issue stages that there are; the rest ask
     int kt = 0;
-    for (; kt + 1 < nk; kt += 2) {
-        step(kt, IC<0>());
-        step(kt + 1, IC<1>());
+    for (; XF32 ? kt / 2 + kWRing - 1 < nws : kt + kS + 1 < nk; kt += 2) {
+        step(kt, IC<0>(), BC<false>());
+        step(kt + 1, IC<1>(), BC<false>());
     }
-    if (kt < nk) step(kt, IC<0>());
+    for (; kt + 1 < nk; kt += 2) {
+        step(kt, IC<0>(), BC<true>());
+        step(kt + 1, IC<1>(), BC<true>());
+    }
+    if (kt < nk) step(kt, IC<0>(), BC<true>());
     // (the products are asm: the wait states between the last and a read of
     // its accumulators are ours to give, and the accumulators pass through
     // what follows the wait, so that no read of them can stand before it)
