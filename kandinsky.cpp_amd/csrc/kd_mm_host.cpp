@@ -5,6 +5,7 @@
 // the call.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "../../include/kd_mm.h"
@@ -103,11 +104,16 @@ size_t ws_bytes(const kd_mm_desc *d) {
 // The tile of a call (32 * (tile / 10) outputs x 32 * (tile % 10) tokens) of
 // more than kMmSkinnyRows tokens: the one whose rounds of workgroups (256 at
 // once, one per CU) take least time.  A round's time with every CU at it, F32
-// x, is `fixed` (first loads, sums and stores) + `us` * K / 4096; with BF16 x
-// all take 0.7-0.9 of that, so their order holds.  Small tiles move more
-// bytes per product, large ones leave CUs idle.  (Without the fixed part
-// calls of few k and many tiles took too small a tile: 5,000 x 4096 x 32
-// 36 us against 28.)
+// x, is `fixed` (first loads, sums and stores) + `us` * K / 4096.  Small tiles
+// move more bytes per product, large ones leave CUs idle.  (Without the fixed
+// part calls of few k and many tiles took too small a tile: 5,000 x 4096 x 32
+// 36 us against 28.)  The large tiles' fixed part is mostly stores, in
+// proportion to the outputs there are (60,000 tokens, K = 32, one round: 8.3
+// us with 4 outputs, 11.0 with 64, 16 with 256; taken as 12 for any, 60,000 x
+// 4 x 32 ran in 32 x 32 tiles, 11.4 us).  The same table serves BF16 x, whose
+// times are 0.4-1.1 of these: over 225 shapes (17 to 63,488 tokens, 4 to
+// 16,384 outputs, K 32 to 16,384) the tile taken is in the mean 1.8% (F32 x)
+// and 0.9% (BF16) slower than the fastest of the nine, at worst 27%.
 int choose_tile(int64_t M, int64_t N, int64_t K) {
     constexpr struct { int tile, n, m; double fixed, us; } kTiles[] = {
         {88, 256, 256, 12.0, 110.0}, {84, 256, 128, 7.0, 69.0}, {44, 128, 128, 6.0, 37.0},
@@ -118,7 +124,8 @@ int choose_tile(int64_t M, int64_t N, int64_t K) {
     for (const auto &t : kTiles) {
         const int64_t tiles = ((N + t.n - 1) / t.n) * ((M + t.m - 1) / t.m);
         if (t.tile != 88 && tiles > kdfa::kMmMaxBlocks) continue;
-        const double cost = (double)((tiles + 255) / 256) * (t.fixed + t.us * (double)K / 4096.0);
+        const double stores = t.n == 256 ? 0.45 + 0.55 * (double)std::min<int64_t>(N, t.n) / t.n : 1.0;
+        const double cost = (double)((tiles + 255) / 256) * (t.fixed * stores + t.us * (double)K / 4096.0);
         if (cost < least) { least = cost; best = t.tile; }
     }
     return best;
