@@ -110,22 +110,27 @@ size_t ws_bytes(const kd_mm_desc *d) {
 // 36 us against 28.)  The large tiles' fixed part is mostly stores, in
 // proportion to the outputs there are (60,000 tokens, K = 32, one round: 8.3
 // us with 4 outputs, 11.0 with 64, 16 with 256; taken as 12 for any, 60,000 x
-// 4 x 32 ran in 32 x 32 tiles, 11.4 us).  The same table serves BF16 x, whose
+// 4 x 32 ran in 32 x 32 tiles, 11.4 us).  And the rounds take no less than x
+// from HBM (5.6 TB/s): then rounds cost their fixed parts only, and the fewest
+// do best (60,000 x 64 x 4096, F32 x, 178 us in one round of 256 x 256, 184 in
+// four of 64 x 64).  The same table serves BF16 x, whose
 // times are 0.4-1.1 of these: over 225 shapes (17 to 63,488 tokens, 4 to
 // 16,384 outputs, K 32 to 16,384) the tile taken is in the mean 1.8% (F32 x)
 // and 0.9% (BF16) slower than the fastest of the nine, at worst 27%.
-int choose_tile(int64_t M, int64_t N, int64_t K) {
+int choose_tile(int64_t M, int64_t N, int64_t K, bool x_f32) {
     constexpr struct { int tile, n, m; double fixed, us; } kTiles[] = {
         {88, 256, 256, 12.0, 110.0}, {84, 256, 128, 7.0, 69.0}, {44, 128, 128, 6.0, 37.0},
         {43, 128, 96, 5.0, 31.0},    {42, 128, 64, 4.0, 23.5},  {23, 64, 96, 3.5, 23.5},
         {22, 64, 64, 2.5, 16.5},     {21, 64, 32, 1.7, 10.8},   {11, 32, 32, 1.2, 7.8}};
+    const double stream = (double)M * (double)K * (x_f32 ? 4 : 2) / 5.6e6;   // us
     int best = 88;
     double least = 1e300;
     for (const auto &t : kTiles) {
         const int64_t tiles = ((N + t.n - 1) / t.n) * ((M + t.m - 1) / t.m);
         if (t.tile != 88 && tiles > kdfa::kMmMaxBlocks) continue;
         const double stores = t.n == 256 ? 0.45 + 0.55 * (double)std::min<int64_t>(N, t.n) / t.n : 1.0;
-        const double cost = (double)((tiles + 255) / 256) * (t.fixed * stores + t.us * (double)K / 4096.0);
+        const double rounds = (double)((tiles + 255) / 256);
+        const double cost = rounds * t.fixed * stores + std::max(rounds * t.us * (double)K / 4096.0, stream);
         if (cost < least) { least = cost; best = t.tile; }
     }
     return best;
@@ -206,7 +211,7 @@ int kd_mm_run(const kd_mm_desc *desc, void *workspace, size_t workspace_bytes, v
         e = kdfa::launch_mm_skinny(a, x_f32, hs);
     } else {
         // (counted in 64 bits: M and N may be within a tile of 2^31)
-        const int tile = choose_tile(M, N, K);
+        const int tile = choose_tile(M, N, K, x_f32);
         const int64_t tiles_n = (N + 32 * (tile / 10) - 1) / (32 * (tile / 10));
         const int64_t tiles_m = (M + 32 * (tile % 10) - 1) / (32 * (tile % 10));
         if (tiles_n * tiles_m > kI32Max) return KD_FA_ERR_SHAPE;

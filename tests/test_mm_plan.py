@@ -17,8 +17,10 @@ def test_sizes_within_a_tile_of_2_31(M, N, K):
     assert p.tiles_m * tm <= 2 ** 31 and p.tiles_n * tn <= 2 ** 31
 
 
-@pytest.mark.parametrize("M,N,K", [(60000, 4, 32), (59971, 24, 64), (60000, 64, 32), (60000, 64, 256)])
+@pytest.mark.parametrize("M,N,K", [(60000, 4, 32), (59971, 24, 64), (60000, 64, 32), (60000, 64, 256),
+                                   (61442, 64, 4096), (60000, 64, 512)])
 def test_few_outputs_of_many_tokens_take_one_round(M, N, K):
     """The large tile's time is mostly stores: with few outputs its one round
-    beats several of small tiles (60,000 x 4 x 32: 8.3 us against 11.4)."""
+    beats several of small tiles (60,000 x 4 x 32: 8.3 us against 11.4), also
+    where x's way from HBM bounds both (60,000 x 64 x 4096: 178 against 184)."""
     assert plan(M, N, K)[:2] == ("mm_bf16", 88)
