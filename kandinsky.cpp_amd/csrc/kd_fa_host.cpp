@@ -609,8 +609,11 @@ int run(const kd_fa_desc *d, const kd_fa_rope *r, const kd_fa_qk_norm *n, void *
     hipStream_t hs = static_cast<hipStream_t>(stream);
     if (d->q.ne[0] == kHeadDimVae) {
         // with a workspace, the key split of short query sets (the partial
-        // results, then the merge into dst)
-        const D512Split sp = d512_split(Lq, a.Lk, H, B, route);
+        // results, then the merge into dst), unless 64-row workgroups give
+        // every CU one without it (256 heads of 32 rows, 256 keys: 28 us,
+        // split 48; KD_FA_ROUTE_D512_R1 looks at 32-row ones)
+        const bool filled = !(route & KD_FA_ROUTE_D512_R1) && (Lq + 63) / 64 * H * B >= 256;
+        const D512Split sp = filled ? D512Split{} : d512_split(Lq, a.Lk, H, B, route);
         const bool split = sp.S > 1 && ws && ws_bytes >= sp.bytes;
         // 64 query rows per workgroup (half the key stream per row, 1.5-1.7
         // times the time) where that saves a round of workgroups, one per

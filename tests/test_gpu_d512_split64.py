@@ -52,3 +52,25 @@ def test_split_64_rows(case):
     rows = np.unique(np.concatenate([rows, [0, B * H * Lq - 1]]))
     ref = orc.fa_f64(q, k, v, scale=D ** -0.5, rows=rows)
     assert_parity(gather_rows(outs[0], rows, H, Lq), ref, f"d512 split 64 rows {case}")
+
+
+@pytest.mark.parametrize("shape", [(1, 256, 32, 256), (4, 64, 31, 520), (2, 128, 17, 130)], ids=lambda s: "x".join(map(str, s)))
+def test_many_short_heads_are_not_split(shape):
+    """One 64-row workgroup per CU or more: the workspace stays untouched and
+    the result is the call's without one."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    B, H, Lq, Lk = shape
+    print(f"[case] d512 short heads {shape}", flush=True)
+    q, k, v = (randn(s, t, i).to(DEV) for i, (s, t) in
+               enumerate([((B, H, Lq, D), torch.float32), ((B, H, Lk, D), torch.float16), ((B, H, Lk, D), torch.float16)]))
+    outs = [torch.empty((B, Lq, H, D), dtype=torch.float32, device=DEV) for _ in range(2)]
+    descs = [kd_fa.make_desc(q, k, v, None, o, D ** -0.5) for o in outs]
+    size = kd_fa.workspace_size_full(descs[0])
+    assert size > 0
+    ws = torch.full((size,), 0x7F, dtype=torch.uint8, device=DEV)
+    assert kd_fa.run_desc(descs[0], workspace=ws) == kd_fa.OK
+    assert kd_fa.run_desc(descs[1]) == kd_fa.OK
+    torch.cuda.synchronize()
+    assert bool((ws == 0x7F).all())
+    assert torch.equal(outs[0], outs[1])
