@@ -32,11 +32,13 @@ def test_k_reads_return_before_the_refill(which):
                 k_reads.update(after)
     assert len(k_reads) == 8 * 3, len(k_reads)   # prologue, the loop's first tile (peeled), the loop
     # K's DMAs: those with the offset registers of the first tile's eight (the
-    # kernel's first DMAs; V's share no register with them)
+    # kernel's first DMAs; V's, the next eight and issued before the first
+    # wait, share no register with them)
     dma = [(i, ln.split()[1]) for i, ln in enumerate(lines) if ln.startswith("buffer_load") and ln.endswith(" lds")]
     k_off = {r for _, r in dma[:8]}
     k_dma = {i for i, r in dma if r in k_off}
-    assert len(k_off) == 8 and not k_off & {r for _, r in dma[16:24]}
+    assert len(k_off) == 8 and not k_off & {r for _, r in dma[8:16]}
+    assert dma[15][0] < min(k_reads)
     assert len(k_dma) == 8 * 5   # the prologue's two tiles, the first tile (peeled), the loop's two branches
     reached = set()
     # state: line, K reads since a marker, LDS operations in flight (True: a read of K), oldest first
@@ -67,3 +69,22 @@ def test_k_reads_return_before_the_refill(which):
             flight = ()
         todo += [(j, read, flight) for j in nxt[i]]
     assert reached == k_dma
+
+
+@pytest.mark.parametrize("which", range(4))
+def test_one_tile_fetches_one_tile(which):
+    """A range of one key tile (a split short call is all such) brings that
+    tile's K and V and nothing else: the fewest DMAs of any path on from the
+    first."""
+    lines = kernels("kd_fa_d512.hip")[_names()[which]]
+    nxt = successors(lines)
+    dma = [ln.startswith("buffer_load") and ln.endswith(" lds") for ln in lines]
+    first = dma.index(True)
+    least, todo = {first: 1}, [first]
+    while todo:
+        i = todo.pop()
+        for j in nxt[i]:
+            if least[i] + dma[j] < least.get(j, len(lines)):
+                least[j] = least[i] + dma[j]
+                todo.append(j)
+    assert min(n for i, n in least.items() if lines[i].startswith("s_endpgm")) == 16
