@@ -21,8 +21,10 @@ CASES = [
     (1, 1, 2100, 2011, torch.bfloat16, torch.float32),
     (1, 1, 4095, 161, torch.float16, torch.float32),
     (2, 3, 1300, 130, torch.float16, torch.float16),
-    (1, 2, 4097, 129, torch.bfloat16, torch.bfloat16),
+    (1, 2, 2600, 193, torch.bfloat16, torch.bfloat16),
 ]
+# too many 32-row blocks for a split: the unsplit call, ragged in rows and keys
+UNSPLIT = (1, 2, 4097, 129, torch.bfloat16, torch.bfloat16)
 
 
 def _wide(x):
@@ -32,7 +34,7 @@ def _wide(x):
     return w[..., :D]
 
 
-@pytest.mark.parametrize("case", CASES, ids=lambda c: f"B{c[0]}H{c[1]}q{c[2]}k{c[3]}{str(c[4])[-4:]}")
+@pytest.mark.parametrize("case", CASES + [UNSPLIT], ids=lambda c: f"B{c[0]}H{c[1]}q{c[2]}k{c[3]}{str(c[4])[-4:]}")
 def test_split_64_rows(case):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
@@ -42,7 +44,9 @@ def test_split_64_rows(case):
     qd, kd, vd = q.to(DEV), _wide(k), _wide(v)
     outs = [torch.empty((B, Lq, H, D), dtype=torch.float32, device=DEV) for _ in range(2)]
     descs = [kd_fa.make_desc(qd, kd, vd, None, o, D ** -0.5) for o in outs]
-    ws = torch.empty(kd_fa.workspace_size_full(descs[0]), dtype=torch.uint8, device=DEV).fill_(0x7F)
+    size = kd_fa.workspace_size_full(descs[0])
+    assert (size > 0) == (case != UNSPLIT)
+    ws = torch.empty(size, dtype=torch.uint8, device=DEV).fill_(0x7F)
     assert kd_fa.run_desc(descs[0], workspace=ws) == kd_fa.OK
     with kd_fa.routing(kd_fa.ROUTE_D512_R1):
         assert kd_fa.run_desc(descs[1], workspace=ws) == kd_fa.OK

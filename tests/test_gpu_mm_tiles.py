@@ -16,21 +16,35 @@ pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
 
-# M, N, K; the tile the choice takes stands beside the larger ones
+# M, N, K (test_mm_plan.py holds the kernel and tile that each takes)
 CASES = [(1, 4, 32), (8, 36, 96), (9, 100, 416), (16, 260, 1184), (3, 16388, 288), (12, 16384, 64),
          (17, 32, 64), (33, 100, 544),
          (31, 8200, 160),     # 64 x 32
          (130, 4100, 96),     # 64 x 64
          (300, 4096, 416),    # 64 x 96
          (850, 2100, 672),    # 128 x 64
-         (700, 4100, 352),    # 128 x 96
-         (1030, 8000, 736),   # 128 x 128
+         (700, 4100, 352),    # 128 x 128
+         (1030, 8000, 736),   # 128 x 96
          (1540, 4100, 96), (1700, 4096, 32), (2047, 4004, 352),   # 256 x 128
          (3900, 4080, 96), (3841, 4064, 64), (4090, 4064, 416)]   # 256 x 256
+# k of several times the stages that the LDS rings hold: every buffer is
+# refilled after it has been read, and the steady loops run; an odd and an
+# even number of 64-k stages, whole and with a half last one
+DEEP = [(M, N, K) for M, N, ks in [
+    (2, 260, (2816, 2848, 2880)), (12, 260, (2816, 2848, 2880)), (2, 16388, (2848, 2880)), (12, 16388, (2848, 2880)),
+    (33, 112, (832, 864, 896, 928)),      # 32 x 32
+    (34, 4144, (832, 864, 896, 928)),     # 64 x 32
+    (99, 4184, (832, 864, 896, 928)),     # 64 x 64
+    (3347, 260, (832, 864, 896, 928)),    # 64 x 96
+    (291, 4148, (832, 864, 928)),         # 128 x 64
+    (3274, 524, (832, 864, 928)),         # 128 x 96
+    (4048, 648, (832, 864, 928)),         # 128 x 128
+    (3601, 1044, (832, 864)),             # 256 x 128
+    (4057, 2180, (832, 864))] for K in ks]   # 256 x 256
 
 
 @pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
-@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("case", CASES + DEEP, ids=lambda c: "x".join(map(str, c)))
 def test_every_tile(case, xdt):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")

@@ -84,3 +84,23 @@ def test_operands_are_not_written_just_ahead_of_a_product(which):
             states += not up.startswith((";", "."))
             if states < 2:
                 todo += [(p, states) for p in before.get(j, [])]
+
+
+@pytest.mark.parametrize("which", range(4))
+def test_every_step_loads_its_share_of_f32_x(which):
+    """The waits count on the loads and DMAs of each step, F32 x's plain loads
+    among them: none merged, dropped or added (two stages ahead of the loop
+    and two behind its first rounding, then one per step of the two loops;
+    the single last step has none)."""
+    name = _instances()[which]
+    lines = kernels("kd_mm_kernel.hip")[name]
+    end = lines.index("; accumulator complete")
+    loads = sum(ln.startswith("global_load_dwordx4") for ln in lines[:end])
+    dmas = sum(ln.startswith("global_load_lds_dwordx4") for ln in lines[:end])
+    mb = 4 if "Li4E" in name else 2
+    if "Lb1E" in name:
+        assert (loads, dmas) == (2 * mb * (4 + 4), 3 * 8 + 5 * 4)
+    else:
+        ahead = (5 if mb == 4 else 6) - 1
+        per = 4 + mb
+        assert (loads, dmas) == (0, ahead * per + (2 + mb // 2) + 5 * per)

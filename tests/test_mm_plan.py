@@ -3,6 +3,7 @@ kd_mm_host.cpp), on the host alone."""
 import pytest
 
 from mm_plan import plan
+from test_gpu_mm_tiles import CASES, DEEP
 
 
 @pytest.mark.parametrize("M,N,K", [(2 ** 31 - 1, 4, 32), (2 ** 31 - 255, 4, 32), (1, 2 ** 31 - 4, 32),
@@ -24,3 +25,42 @@ def test_few_outputs_of_many_tokens_take_one_round(M, N, K):
     beats several of small tiles (60,000 x 4 x 32: 8.3 us against 11.4), also
     where x's way from HBM bounds both (60,000 x 64 x 4096: 178 against 184)."""
     assert plan(M, N, K)[:2] == ("mm_bf16", 88)
+
+
+# the tile (outputs, tokens in units of 32) of test_gpu_mm_tiles.py's cases of more than 16 tokens
+TILE = {(17, 32): 11, (33, 100): 11, (31, 8200): 21, (130, 4100): 22, (300, 4096): 23, (850, 2100): 42, (700, 4100): 44,
+        (1030, 8000): 43, (1540, 4100): 84, (1700, 4096): 84, (2047, 4004): 84, (3900, 4080): 88, (3841, 4064): 88,
+        (4090, 4064): 88,
+        (33, 112): 11, (34, 4144): 21, (99, 4184): 22, (3347, 260): 23, (291, 4148): 42, (3274, 524): 43, (4048, 648): 44,
+        (3601, 1044): 84, (4057, 2180): 88}
+LDS = 160 * 1024
+
+
+def _stages(tile, x_f32):
+    """LDS stages of an mm_ksplit instance, as the kernel sizes its ring."""
+    return min(5, LDS // (tile // 10 * 4096 + tile % 10 * 32 * (256 if x_f32 else 128)))
+
+
+@pytest.mark.parametrize("x_f32", [True, False], ids=["f32", "bf16"])
+def test_gpu_cases_take_their_tiles(x_f32):
+    for M, N, K in CASES + DEEP:
+        p = plan(M, N, K, x_f32)
+        assert (p.kernel == "mm_skinny") == (M <= 16)
+        assert M <= 16 or p.tile == TILE[M, N], (M, N, K, p)
+    # every instance runs its steady loop and refills every buffer of its ring
+    deep = {}
+    for M, N, K in DEEP:
+        nk = -(-K // 64)
+        if M <= 16:
+            wide = -(-N // 64) >= 256
+            stages = {(True, 8): 4, (False, 8): 3, (True, 16): 3, (False, 16): 5}[wide, 8 if M <= 8 else 16]
+            assert nk // 4 >= 2 * stages + 1
+            deep.setdefault((wide, M <= 8), set()).add(K % 64)
+        else:
+            tile = TILE[M, N]
+            if tile < 84:
+                assert nk >= 2 * _stages(tile, x_f32) + 3
+            else:
+                assert K // 32 >= 2 * 6 + 3
+            deep.setdefault(tile, set()).add(K % 64)
+    assert len(deep) == 4 + 9 and all(k == {0, 32} for k in deep.values())
