@@ -112,17 +112,19 @@ size_t ws_bytes(const kd_mm_desc *d) {
 // us with 4 outputs, 11.0 with 64, 16 with 256; taken as 12 for any, 60,000 x
 // 4 x 32 ran in 32 x 32 tiles, 11.4 us).  And the rounds take no less than x
 // from HBM (5.6 TB/s): then rounds cost their fixed parts only, and the fewest
-// do best (60,000 x 64 x 4096, F32 x, 178 us in one round of 256 x 256, 184 in
-// four of 64 x 64).  The same table serves BF16 x, whose
-// times are 0.4-1.1 of these: over 225 shapes (17 to 63,488 tokens, 4 to
+// do best (60,000 x 64 x 512, F32 x, 27.0 us in one round of 256 x 256, 28.9
+// in four of 64 x 64).  F32 x and BF16 x take the same tile, so that F32 x has
+// the bits of its rounding: the table is F32 x's, the stream BF16 x's (with
+// F32 x's 61,442 x 64 x 4096 would gain 3% at F32 x and lose 19% at BF16).
+// BF16 x's times are 0.4-1.1 of the table's: over 225 shapes (17 to 63,488 tokens, 4 to
 // 16,384 outputs, K 32 to 16,384) the tile taken is in the mean 1.8% (F32 x)
 // and 0.9% (BF16) slower than the fastest of the nine, at worst 27%.
-int choose_tile(int64_t M, int64_t N, int64_t K, bool x_f32) {
+int choose_tile(int64_t M, int64_t N, int64_t K) {
     constexpr struct { int tile, n, m; double fixed, us; } kTiles[] = {
         {88, 256, 256, 12.0, 110.0}, {84, 256, 128, 7.0, 69.0}, {44, 128, 128, 6.0, 37.0},
         {43, 128, 96, 5.0, 31.0},    {42, 128, 64, 4.0, 23.5},  {23, 64, 96, 3.5, 23.5},
         {22, 64, 64, 2.5, 16.5},     {21, 64, 32, 1.7, 10.8},   {11, 32, 32, 1.2, 7.8}};
-    const double stream = (double)M * (double)K * (x_f32 ? 4 : 2) / 5.6e6;   // us
+    const double stream = (double)M * (double)K * 2.0 / 5.6e6;   // us
     int best = 88;
     double least = 1e300;
     for (const auto &t : kTiles) {
@@ -211,7 +213,7 @@ int kd_mm_run(const kd_mm_desc *desc, void *workspace, size_t workspace_bytes, v
         e = kdfa::launch_mm_skinny(a, x_f32, hs);
     } else {
         // (counted in 64 bits: M and N may be within a tile of 2^31)
-        const int tile = choose_tile(M, N, K, x_f32);
+        const int tile = choose_tile(M, N, K);
         const int64_t tiles_n = (N + 32 * (tile / 10) - 1) / (32 * (tile / 10));
         const int64_t tiles_m = (M + 32 * (tile % 10) - 1) / (32 * (tile % 10));
         if (tiles_n * tiles_m > kI32Max) return KD_FA_ERR_SHAPE;

@@ -75,6 +75,21 @@ def test_every_tile(case, xdt):
     assert np.array_equal(out.cpu().numpy(), got.numpy())
 
 
+@pytest.mark.parametrize("case", [(2, 260, 2848), (33, 112, 864), (99, 4184, 96), (300, 4096, 416), (1540, 4100, 96),
+                                  (4057, 2180, 832)], ids=lambda c: "x".join(map(str, c)))
+def test_f32_x_has_the_bits_of_its_rounding(case):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    M, N, K = case
+    print(f"[case] mm x types {case}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    w = (torch.randn((N, K), generator=g) * 0.05).bfloat16().to(DEV)
+    x = torch.randn((M, K), generator=g).to(DEV)
+    outs = [kd_mm.linear(v, w) for v in (x, x.bfloat16())]
+    torch.cuda.synchronize()
+    assert torch.equal(*outs)
+
+
 @pytest.mark.parametrize("shape", [(1, 32), (3, 96), (71, 352), (129, 4096)], ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("kind", ["q8_0", "q4_0", "bf16", "f16", "f32"])
 def test_dequant_padded_rows(kind, shape):
