@@ -20,7 +20,11 @@
  * d * q for Q8_0, d * (nibble - 8) for Q4_0, exactly as ggml's
  * dequantize_row_q8_0 / _q4_0 compute it in F32), x is rounded to BF16,
  * the products are accumulated in F32 on the matrix cores, the bias is
- * added in F32.  ggml's own CPU path instead rounds x to Q8_0 blocks; both
+ * added in F32.  The order of a row's F32 sum depends on M, N and K (few
+ * tokens are summed in four parts, many in one), not on x's type: equal calls
+ * give equal bits, and F32 x those of its BF16 rounding, but a token's result
+ * may differ in its last bits between calls of other sizes, for instance
+ * alone and in a batch.  ggml's own CPU path instead rounds x to Q8_0 blocks; both
  * stay within the rounding of the 8-bit formats of the exact product.
  *
  * All device pointers belong to the caller; nothing is allocated, freed,

@@ -39,9 +39,12 @@ namespace kdfa {
 // With a key split (a.n_split > 1, short query sets with a workspace), a
 // workgroup runs only its range of key tiles and leaves the unnormalised O,
 // running max and row sum of its rows for d512_combine.
-// What binds is LDS: at R = 2 a tile moves 212 KB through it (1,650 of its
-// about 2,900 cycles; the products take 1,024).  F16 K / V: 4,096 tokens with
-// the key split 96.8 -> 73.4 us, 8,192 311 -> 205, 16,384 924 -> 706; with
+// LDS is the busiest unit by count: at R = 2 a tile moves 212 KB through it
+// (1,650 of its about 2,900 cycles; the products take 1,024).  No unit is at
+// its limit: at 4,096 tokens the matrix cores are busy 24% of the time, 15%
+// of the waves' time waits for an LDS instruction (conflicts: 3.7%), and the
+// rest is the chain of a step with one wave per SIMD.  F16 K / V: 4,096 tokens
+// with the key split 96.8 -> 72.6 us, 8,192 311 -> 203, 16,384 924 -> 706; with
 // the products in sequence with the exchange and the DMAs in one burst
 // before the barrier 16,384 tokens took 880.
 constexpr int kD5 = 512;                     // D, four 128-column slices

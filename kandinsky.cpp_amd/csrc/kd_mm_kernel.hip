@@ -167,16 +167,20 @@ hipError_t launch_dequant(const DqArgs &a, hipStream_t s) {
 // from the L2 twice (from every CU, rows of 64 bytes arrive at 65 KB per
 // microsecond and CU, of 128 at 128; 16,000 x 4096 x 16384 2.11 -> 1.85 ms).
 // In LDS 16-byte chunk c of row r lies at c ^ ((r >> 2) & 3) (of a 128-byte
-// row, at c ^ ((r >> 1) & 7)): the 16 rows that 16 lanes of an operand read
-// touch fill the 64 banks once.
+// row, at c ^ ((r >> 1) & 7)), which spreads the 16 rows of an operand read
+// over the 64 banks.  The 64-byte rows still conflict (F32 x, 63,488 tokens:
+// 7.5% of the cycles: the 16-byte reads are served for lanes 0-3, 12-15,
+// 20-27 together, not for 16 in a row); a swizzle without conflicts did not
+// change the time.
 //
 // Per stage a wave reads 8 W and 2 MB X fragments and issues 16 MB MFMAs in
 // two halves (all W against half of X); the fragment reads of what follows,
 // the DMAs of a later stage and X's loads, roundings and LDS writes are
 // spread over them one by one (the reads in one burst behind the barrier:
 // 10% more at BF16 x); the one barrier, between the halves, publishes the
-// next stage.  The loop has no conditions: past the last stage the DMAs and
-// loads bring the last one again.
+// next stage.  The loop has no conditions; the last steps, apart, issue as
+// many operations, all of one chunk where there is no stage left (bringing
+// the last stage again cost 2-6% at K = 64, 1-4% at 4096).
 //
 // 63,488 x 4096 x 4096: F32 x 2.30 -> 1.99 ms, BF16 x 1.89 -> 1.69 ms
 // against 32 x 32 x 16 products with F32 X read from LDS; 4,000 tokens, F32
@@ -195,9 +199,9 @@ void mm_bf16(MmArgs a) {
     typedef E::vec8 vec8;
     constexpr int BM = 64 * MB;
     constexpr int kXTile = BM * 64;                        // BF16 X rows of a stage
-    constexpr int kS = XF32 ? 6 : MB == 4 ? 5 : 6;         // stages of W (and BF16 X) in LDS
+    constexpr int kS = MB == 4 ? 5 : 6;                    // BF16 X: stages of W and X in LDS
     constexpr int kWRing = 4;                              // F32 X: double stages of W (128-byte rows)
-        constexpr int kXC = 2 * MB;                            // F32 X: 16-byte loads of a thread per stage
+    constexpr int kXC = 2 * MB;                            // F32 X: 16-byte loads of a thread per stage
     constexpr int kXD = XF32 ? 0 : MB;                     // BF16 X: DMAs of a wave per stage
     constexpr int kVm = 4 + (XF32 ? kXC : kXD);            // vector memory operations of a wave per stage
     constexpr int kX0 = XF32 ? kWRing * 2 * kMmWTile : kS * kMmWTile;   // the X buffers behind W's
@@ -348,7 +352,7 @@ void mm_bf16(MmArgs a) {
         else
             dma_j(dk + kS - 2, dbuf, kWork0 + slot, end_c);
     };
-    // (as many stages as there are: with two, four took 5% of the call)
+    // (as many stages as there are)
     if constexpr (XF32) {
 #pragma unroll
         for (int s = 0; s < kWRing - 1; ++s)
@@ -378,7 +382,7 @@ void mm_bf16(MmArgs a) {
         }
     }
 #pragma unroll
-    for (int slot = 0; slot < kWork0; ++slot) work0(slot, 1, kS - 1, IC<1>(), BC<true>());
+    for (int slot = 0; slot < kWork0; ++slot) work0(slot, 1, kS - 1, IC<1>(), BC<true>());   // (F32 X: no buffer)
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 8; ++i) read_a(0, IC<0>(), i);

@@ -40,9 +40,9 @@ static __device__ __forceinline__ bf16x8 round8(f32x4 u, f32x4 v) {
 }
 
 // LDS rows of one stage hold 64 k: 128 bytes of BF16 (16-byte chunk c of row
-// r at c ^ ((r >> 1) & 7)) or 256 bytes of F32 (at c ^ (r & 15)), so that
-// the 16 rows that 16 lanes of an operand read touch lie in 16 different
-// groups of four banks.
+// r at c ^ ((r >> 1) & 7)) or 256 bytes of F32 (at c ^ (r & 15)), which
+// spreads the rows of an operand read over the banks (conflicts: 0.5% of
+// mm_skinny's cycles, 1.3-1.9% of mm_ksplit's).
 static __device__ __forceinline__ int swz16(int r) { return (r >> 1) & 7; }
 static __device__ __forceinline__ int swz32(int r) { return r & 15; }
 
@@ -51,8 +51,8 @@ static __device__ __forceinline__ int swz32(int r) { return r & 15; }
 // the stream of W from HBM.  A wave takes stages wave, wave + 4, ... of 64 k
 // (whole 128-byte lines of W) and keeps S - 1 of them in flight by itself,
 // 64-80 KB of W per CU; rows of X past M repeat the last one.  2 x 16384 x
-// 4096, BF16 W, F32 x: 118.5 -> 29.5 us (4.6 TB/s; mm_bf16 ran 64
-// workgroups); 2 x 4096 x 4096 116 -> 11.9, 2 x 4096 x 16384 437 -> 33.5,
+// 4096, BF16 W, F32 x: 118.5 -> 29.5 us (26.6 in the kernel, W fetched once
+// at 5.0 TB/s; mm_bf16 ran 64 workgroups); 2 x 4096 x 4096 116 -> 11.9, 2 x 4096 x 16384 437 -> 33.5,
 // 16 x 4096 x 16384 458 -> 43.
 // ---------------------------------------------------------------------------
 template <int NB, int XR, int S, bool XF32>
@@ -174,8 +174,11 @@ __global__ __launch_bounds__(256) void mm_skinny(MmArgs a) {
 // mm_ksplit: 32 NB outputs x 32 MB tokens per workgroup.  Splitting k over
 // the waves lets each read every W and X row of the tile once per 16 k: half
 // the LDS reads of a 2 x 2 grid of waves, which would bind at these sizes.
-// What binds is the stage's way into LDS (64 B/clk per CU, F32 x twice the
-// bytes of BF16) and its reads.  F32 x, N = K = 4096: 64 tokens 127 -> 15.8
+// What takes most is the stages' way into LDS (64 B/clk per CU, F32 x twice
+// the bytes of BF16): 16 of the kernel's 29 us at 300 tokens, 39 of 70 at
+// 1,280, at the 134 KB per microsecond and CU that a probe reached; the matrix
+// cores are busy 21 and 31% of the time, and 6 and 10% of the waves' time
+// waits for an LDS instruction.  F32 x, N = K = 4096: 64 tokens 127 -> 15.8
 // us (1 x 1 blocks), 300 131 -> 28.0 (2 x 3), 600 130 -> 37.8 (4 x 3), 1,280
 // 131 -> 75, 2,000 131 -> 95 (4 x 4), weights from HBM on every call.
 // ---------------------------------------------------------------------------
@@ -190,9 +193,8 @@ void mm_ksplit(MmArgs a) {
     constexpr int kFit = 163840 / kStage;
     constexpr int S = kFit < 5 ? kFit : 5;
     constexpr int kEpi = MB * 16384;              // the four waves' 32 outputs of every token
-    constexpr int kEB = 2 * kEpi <= 163840 ? 2 : 1;
-    constexpr int kLds = S * kStage > kEB * kEpi ? S * kStage : kEB * kEpi;
-    static_assert(S >= 2, "two stages at least");
+    constexpr int kLds = S * kStage > 2 * kEpi ? S * kStage : 2 * kEpi;
+    static_assert(S >= 2 && 2 * kEpi <= 163840, "two stages, and two blocks of sums, at least");
     __shared__ __attribute__((aligned(1024))) char lds[kLds];
     lds_t *const sbase = LDS_PTR(char, lds);
 
@@ -343,8 +345,7 @@ void mm_ksplit(MmArgs a) {
     __syncthreads();
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-        lds_t *const so = sbase + (kEB == 2 ? (nb & 1) * kEpi : 0);
-        if (kEB == 1 && nb > 0) __syncthreads();
+        lds_t *const so = sbase + (nb & 1) * kEpi;
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
