@@ -41,10 +41,13 @@ DEEP = [(M, N, K) for M, N, ks in [
     (4048, 648, (832, 864, 928)),         # 128 x 128
     (3601, 1044, (832, 864)),             # 256 x 128
     (4057, 2180, (832, 864))] for K in ks]   # 256 x 256
+# the large tiles' last steps, apart from their loop, with every number of
+# stages up to those that the loop begins with: 256 x 256, 256 x 128
+ENDS = [(M, N, K) for M, N in ((33001, 132), (1540, 4100)) for K in range(32, 321, 32)]
 
 
 @pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
-@pytest.mark.parametrize("case", CASES + DEEP, ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("case", CASES + DEEP + ENDS, ids=lambda c: "x".join(map(str, c)))
 def test_every_tile(case, xdt):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")

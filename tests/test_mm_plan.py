@@ -6,7 +6,7 @@ import random
 import pytest
 
 from mm_plan import plan
-from test_gpu_mm_tiles import CASES, DEEP
+from test_gpu_mm_tiles import CASES, DEEP, ENDS
 
 
 @pytest.mark.parametrize("M,N,K", [(2 ** 31 - 1, 4, 32), (2 ** 31 - 255, 4, 32), (1, 2 ** 31 - 4, 32),
@@ -47,7 +47,7 @@ def test_both_types_of_x_take_the_same_tile():
 TILE = {(17, 32): 11, (33, 100): 11, (31, 8200): 21, (130, 4100): 22, (300, 4096): 23, (850, 2100): 42, (700, 4100): 44,
         (1030, 8000): 43, (1540, 4100): 84, (1700, 4096): 84, (2047, 4004): 84, (3900, 4080): 88, (3841, 4064): 88,
         (4090, 4064): 88,
-        (33, 112): 11, (34, 4144): 21, (99, 4184): 22, (3347, 260): 23, (291, 4148): 42, (3274, 524): 43, (4048, 648): 44,
+        (33001, 132): 88, (33, 112): 11, (34, 4144): 21, (99, 4184): 22, (3347, 260): 23, (291, 4148): 42, (3274, 524): 43, (4048, 648): 44,
         (3601, 1044): 84, (4057, 2180): 88}
 LDS = 160 * 1024
 
@@ -59,7 +59,7 @@ def _stages(tile, x_f32):
 
 @pytest.mark.parametrize("x_f32", [True, False], ids=["f32", "bf16"])
 def test_gpu_cases_take_their_tiles(x_f32):
-    for M, N, K in CASES + DEEP:
+    for M, N, K in CASES + DEEP + ENDS:
         p = plan(M, N, K, x_f32)
         assert (p.kernel == "mm_skinny") == (M <= 16)
         assert M <= 16 or p.tile == TILE[M, N], (M, N, K, p)
